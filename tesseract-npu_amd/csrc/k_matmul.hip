@@ -39,6 +39,8 @@ namespace tsr {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 // Raw buffer loads over a window of bytes: 32-bit offsets (a vector part and a scalar part), and
 // a load at or past the window's end returns 0.
@@ -191,12 +193,15 @@ __global__ __launch_bounds__(1024, 8) void k_mm_q80(MmArgs a) {
 //   S_j  = v_mfma_i32_32x32x32_i8(X sub-block j, W sub-block j), j = 0..7: the lane's 16-byte
 //          piece 2g + h of the weight row holds values 16 h .. 16 h + 15 of sub-block 2g in its low
 //          nibbles and of sub-block 2g + 1 in its high nibbles;
-//   isum = sum_j sc_j S_j (one v_mad_i32_i24 per output and sub-block);
-//   msum = four v_mfma_f32_32x32x2f32 over k = j of bs_j[token] m_j[row]: every product and every
-//          partial sum is an integer below 2^24 in magnitude (|bs_j| <= 32 * 128, m_j < 64), so the
-//          matrix core's f32 sum is the exact integer (an exact zero may come out as -0 where the
-//          spec's f32(msum) is +0: that can only change the sign of a zero product or term, and a
-//          zero term added to a partial that starts at +0 never changes it);
+//   isum = sum_j sc_j S_j: sc_j = 8 a_j + b_j (a_j, b_j <= 7), the lane's quants multiplied bytewise by
+//          a_j and by b_j (<= 105, an int8 operand), so two chains over the 8 sub-blocks accumulate
+//          A = sum (q a) x and B = sum (q b) x exactly in int32, isum = 8 A + B;
+//   msum = one v_mfma_f32_32x32x16_f16 over the 16 products of (h_j, l_j)[token] and (64 m_j, m_j)[row],
+//          bs_j = 64 h_j + l_j: every operand is an f16 integer, every product and partial sum an integer
+//          below 2^24 in magnitude (|bs_j| <= 32 * 128, m_j < 64), so the f32 sum is the exact integer (an
+//          exact zero may come out as -0 where the spec's f32(msum) is +0: that can only change the sign
+//          of a zero product or term, and a zero term added to a partial that starts at +0 never changes
+//          it). Four v_mfma_f32_32x32x2f32 took 256 cycles for it, this one 32;
 //   term and partial sum on the VALU. Dx is an A256 scale (any f32): while every Dx a wave has met
 //   is 0 or >= 2^-60 in magnitude the plain IEEE operations are the spec operations (see
 //   k_matvec.hip); from the first super-block with a smaller nonzero Dx on, the wave uses the spec
@@ -204,13 +209,14 @@ __global__ __launch_bounds__(1024, 8) void k_mm_q80(MmArgs a) {
 
 // QACT A256 of T token rows, block-major: one aligned 16-lane row per (token, super-block)
 // (qact_a256_row: lane i holds values 16 i .. 16 i + 15, half i & 1 of sub-block i / 2). Writes
-// the quants xq [K/32][T][32 B], the sub-block sums xs [K/32][T] and the scales xd [K/256][tp]
+// the quants xq [K/32][T][32 B], the sub-block sums xs [K/256][T][8] as f16 pairs (h, l) with
+// sum = 64 h + l (l in -32 .. 31, |h| <= 64: both exact) and the scales xd [K/256][tp]
 // (tp >= T, a multiple of 32; tokens T .. tp - 1 get d = 0). Every lane of a wave stays active
 // (the row operations need them): lanes past the last pair quantize a copy and store nothing. Pairs
 // run token-fastest (a wave's 4 rows write the quants of 4 consecutive tokens); the host keeps
 // tp (K / 256) 16 below 2^32.
 __global__ __launch_bounds__(256) void k_qact_mm4(const float * x, uint64_t x_stride, uint32_t K, uint32_t T,
-                                                  uint32_t tp, uint8_t * xq, int32_t * xs, float * xd) {
+                                                  uint32_t tp, uint8_t * xq, uint32_t * xs, float * xd) {
     const uint32_t nsb = K >> 8;
     const uint32_t pair = (blockIdx.x * blockDim.x + threadIdx.x) >> 4;   // (super-block, token < tp)
     const uint32_t l16 = threadIdx.x & 15u;
@@ -231,7 +237,11 @@ __global__ __launch_bounds__(256) void k_qact_mm4(const float * x, uint64_t x_st
         if (t < T) {
             const uint32_t j = 8u * sb + (l16 >> 1);
             *(uint4 *)(xq + ((size_t)j * T + t) * 32u + 16u * (l16 & 1u)) = q;
-            if ((l16 & 1u) == 0u) xs[(size_t)j * T + t] = bs;
+            if ((l16 & 1u) == 0u) {
+                const int bh = (bs + 32) >> 6;
+                const h2_t hl = { (_Float16)bh, (_Float16)(bs - 64 * bh) };
+                xs[((size_t)sb * T + t) * 8u + (l16 >> 1)] = __builtin_bit_cast(uint32_t, hl);
+            }
         }
         if (l16 == 0u) xd[(size_t)sb * tp + t] = t < T ? d : 0.0f;
     }
@@ -241,18 +251,35 @@ __device__ __forceinline__ uint32_t q4k_sc(const uint4 mt, uint32_t j) {
     // meta bytes 4 + j: sc_j | (m_j & 3) << 6; nibble j of bytes 12..15: m_j >> 2 (wlayout.hpp)
     return __builtin_amdgcn_ubfe(j < 4u ? mt.y : mt.z, 8u * (j & 3u), 6);
 }
-__device__ __forceinline__ uint32_t q4k_m(const uint4 mt, uint32_t j) {
-    return __builtin_amdgcn_ubfe(j < 4u ? mt.y : mt.z, 8u * (j & 3u) + 6u, 2) | (__builtin_amdgcn_ubfe(mt.w, 4u * j, 4) << 2);
-}
-
-// GLU: weight rows 2j and 2j + 1 are the gate and up rows of output j; their results are in adjacent
-// lanes of the output phase and y[j] = SWIGLU(gate, up) (as the matvec's GLU epilogue).
-// Without GLU, at most 128 VGPRs: two workgroups share a compute unit (measured faster); the GLU form's
-// epilogue would spill there, and it keeps one.
+// Work split. A workgroup of 4 waves computes a tile of 32 weight rows x 32 tokens. Wave j runs over the
+// super-blocks of PG = 4 consecutive partials, which are consecutive slots of the weight layout, and folds
+// each finished partial into its subtree of the 16-partial tree, parking the left halves of the two open
+// levels in LDS; the four subtrees meet in LDS at the end. (An empty partial is +0, and a sum that starts
+// at +0 is never -0, so folding one in changes nothing. With at most 8 or 4 super-blocks the higher
+// partials are empty, and PG shrinks so that every wave has work.) Eight waves with two partials each and
+// all 16 partials in LDS, as this kernel had it, left a wave two super-blocks to set up and finish for and
+// every load to wait for.
+//
+// Loads. A register is requested again for the next super-block right behind its last use, so that a load
+// has a super-block's work (~3 waves on the SIMD) to arrive. Every load is made on every path and in one
+// order (the scheduling barriers): the counted waits then cover the loads they are for and no others, and
+// no register with a load in flight is copied.
+//
+// What bounds it (512 x 28672 x 4096 with GLU, counters): the VALU, ~84% busy: per tile and super-block 96
+// instructions for the terms (6 per output), ~150 to unpack and scale the weight quants, the rest set-up
+// and epilogue; the matrix cores 30%. Measured, before -> now: that shape 360 -> 250 us, 100 x 4096 x 4096
+// 16.6 -> 15.6, a Llama-3-8B layer over 300 tokens 537 -> 463. Splitting the partials over 2 waves or 1
+// instead of 4 gave 239 / 265 us there and 20 / 36 us at 100 tokens; 64 tokens a wave (unpacked weights used
+// twice) 328 us at the 2 waves a SIMD that its registers leave.
+//
+// GLU: weight rows 2j and 2j + 1 are the gate and up rows of output j, in adjacent lanes: the even lane
+// forms y = SWIGLU(gate, up) of the even tokens, the odd lane of the odd ones.
+constexpr uint32_t kMm4Waves = 4;
 template <bool GLU>
-__global__ __launch_bounds__(512, GLU ? 2 : 4) void k_mm_q4k(MmArgs a) {
-    __shared__ float s_p[16][1024];                                // partial pj of output (r, lane)
-    __shared__ int s_slow[8];
+__global__ __launch_bounds__(64 * kMm4Waves, 3) void k_mm_q4k(MmArgs a) {
+    constexpr int kLev = 2;                                        // open tree levels of a wave
+    __shared__ float4 s_p[kMm4Waves][kLev][4][64];                 // wave, level: values r = 4 q + e of a lane
+    __shared__ int s_slow[kMm4Waves];
     const WGeom g = wgeom(a.N, a.K >> 8, a.rb, true);
     const uint32_t lane = __lane_id(), j = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     uint32_t tx, ty;
@@ -269,48 +296,65 @@ __global__ __launch_bounds__(512, GLU ? 2 : 4) void k_mm_q4k(MmArgs a) {
     const uint64_t wend = B1 + 1u < g.nblk ? (uint64_t)(B1 + 1u) * g.bstride : wl_bytes(g);
     const __amdgpu_buffer_rsrc_t rw = brsrc(a.w + wbase, (uint32_t)(wend - wbase));
     const __amdgpu_buffer_rsrc_t rx = brsrc(a.qa, a.d_off + 4u * a.tp * g.nb);
-    const uint32_t owq = (uint32_t)(wl_quant_off(g, B, R, h, 0u, rr) - wbase);   // piece 2 gg + h: + 16 R (2 gg nb + sl)
-    const uint32_t owm = (uint32_t)(wl_meta_off(g, B, R, 0u, rr) - wbase);       // + 16 R sl
+    const uint32_t np = g.nb > 8u ? 16u : (g.nb > 4u ? 8u : (g.nb > 2u ? 4u : g.nb));   // partials in use, a power of two
+    const uint32_t PG = max(np / kMm4Waves, 1u), w0 = PG * j;
+    const uint32_t sl0 = wl_slot(g, min(w0, 15u), 0u);
     const uint32_t sR = 16u * R, sG = 32u * R * g.nb;
-    const uint32_t ox = 32u * t + 16u * h;                        // quants of sub-block jb: + 32 T jb
-    const uint32_t obs = a.s_off + 4u * t + 4u * a.T * h;         // sums of sub-block 2 q + h: + 4 T 2 q
+    uint32_t owq = (uint32_t)(wl_quant_off(g, B, R, h, sl0, rr) - wbase);   // piece 2 gg + h: + sG gg; + sR per slot
+    uint32_t owm = (uint32_t)(wl_meta_off(g, B, R, sl0, rr) - wbase);
+    const uint32_t ox = 32u * t + 16u * h;                         // quants of sub-block jb: + 32 T jb
+    const uint32_t obs = a.s_off + 32u * t + 16u * h;              // sums (h_j, l_j), j = 4 h ..: + 32 T s
     const uint32_t odx = h ? 0x80000000u : a.d_off + 4u * (t0 + c);   // token t0 + c's scale: + 4 tp s
-    const uint32_t m4 = 0x0F0F0F0Fu;
+    const uint32_t m4 = 0x0F0F0F0Fu, T32 = 32u * a.T;
     typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
     // byte-wise q * f of a dword of quants q <= 15 and f <= 7 (no byte carries into the next: q f <= 105)
     auto bmul = [](uint32_t q, uint32_t f) -> int {
         return (int)__builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, q) * (u16x2){(unsigned short)f, (unsigned short)f});
     };
+    v4i wv[4], xv[8];                                              // the operands of one super-block
+    v8h bs;
+    float dxl;
+    uint4 mt;
+    auto load_g = [&](uint32_t s, uint32_t gg) {
+        wv[gg] = bload128(rw, owq + sG * gg, 0u);
+#pragma unroll
+        for (uint32_t e = 0; e < 2u; ++e) xv[2u * gg + e] = bload128(rx, ox, T32 * (8u * s + 2u * gg + e));
+    };
+    auto load_t = [&]() { mt = __builtin_bit_cast(uint4, bload128(rw, owm, 0u)); };
+    auto load_m = [&](uint32_t s) {
+        bs = __builtin_bit_cast(v8h, bload128(rx, obs, T32 * s));
+        dxl = bloadf(rx, odx, 4u * a.tp * s);
+    };
     bool slow = false;
-    // wave j computes partials j and j + 8 (8 waves of up to 256 VGPRs)
-    for (uint32_t half = 0; half < 2u; ++half) {
-    const uint32_t pj = j + 8u * half, cnt = wl_count(g, pj), sl0 = wl_slot(g, pj, 0u);
     v16f p;
+    uint32_t left = 0;                                             // super-blocks of this wave still to come
+    for (uint32_t pi = 0; pi < PG; ++pi) left += wl_count(g, w0 + pi);
+    if (left > 0u) {
+        load_t();
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int r = 0; r < 16; ++r) p[r] = 0.0f;
+        for (uint32_t gg = 0; gg < 4u; ++gg) load_g(w0, gg);       // in the loop's order (the waits count loads)
+        __builtin_amdgcn_sched_barrier(0);
+        load_m(w0);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    for (uint32_t pi = 0; pi < PG; ++pi) {
+    const uint32_t pj = w0 + pi, cnt = wl_count(g, pj);
+    p = (v16f){};
     for (uint32_t k = 0; k < cnt; ++k) {
-        const uint32_t sl = sl0 + k, s = pj + 16u * k;
-        v4i wv[4], xv[8];
-#pragma unroll
-        for (uint32_t gg = 0; gg < 4u; ++gg) wv[gg] = bload128(rw, owq + sR * sl + sG * gg, 0u);
-        const uint4 mt = __builtin_bit_cast(uint4, bload128(rw, owm + sR * sl, 0u));
-#pragma unroll
-        for (uint32_t jb = 0; jb < 8u; ++jb) xv[jb] = bload128(rx, ox, 32u * a.T * (8u * s + jb));
-        float bsf[4];
-#pragma unroll
-        for (uint32_t q = 0; q < 4u; ++q) bsf[q] = (float)(int)__builtin_amdgcn_raw_buffer_load_b32(rx, (int)obs, (int)(4u * a.T * (8u * s + 2u * q)), 0);
-        const float dxl = bloadf(rx, odx, 4u * a.tp * s);
-
-        v16f ms = {};
-#pragma unroll
-        for (uint32_t q = 0; q < 4u; ++q)
-            ms = __builtin_amdgcn_mfma_f32_32x32x2f32(bsf[q], (float)q4k_m(mt, 2u * q + h), ms, 0, 0, 0);
-        // isum = sum_j sc_j S_j on the matrix core: sc_j = 8 a_j + b_j (a_j, b_j <= 7), the weight quants
-        // scaled by a_j and by b_j (<= 105: int8) into two exact int32 accumulators, isum = 8 A + B
+        const uint32_t s = pj + 16u * k;
+        --left;
+        // the next super-block (the last one again when there is none: a valid load that nothing uses)
+        const uint32_t sn = left == 0u ? s : (k + 1u < cnt ? s + 16u : pj + 1u);
+        if (left > 0u) { owq += sR; owm += sR; }
+        const uint4 mc = mt;
+        __builtin_amdgcn_sched_barrier(0);                         // (a load in flight shares no register with a live value)
+        load_t();
+        __builtin_amdgcn_sched_barrier(0);
         v16i ia = {}, ib = {};
 #pragma unroll
         for (uint32_t gg = 0; gg < 4u; ++gg) {
-            const uint32_t sc0 = q4k_sc(mt, 2u * gg), sc1 = q4k_sc(mt, 2u * gg + 1u);
+            const uint32_t sc0 = q4k_sc(mc, 2u * gg), sc1 = q4k_sc(mc, 2u * gg + 1u);
             v4i la, lb, ha, hb;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -320,19 +364,30 @@ __global__ __launch_bounds__(512, GLU ? 2 : 4) void k_mm_q4k(MmArgs a) {
                 ha[e] = bmul(hi, sc1 >> 3);
                 hb[e] = bmul(hi, sc1 & 7u);
             }
-            ia = __builtin_amdgcn_mfma_i32_32x32x32_i8(xv[2 * gg], la, ia, 0, 0, 0);
-            ib = __builtin_amdgcn_mfma_i32_32x32x32_i8(xv[2 * gg], lb, ib, 0, 0, 0);
-            ia = __builtin_amdgcn_mfma_i32_32x32x32_i8(xv[2 * gg + 1], ha, ia, 0, 0, 0);
-            ib = __builtin_amdgcn_mfma_i32_32x32x32_i8(xv[2 * gg + 1], hb, ib, 0, 0, 0);
+            ia = __builtin_amdgcn_mfma_i32_32x32x32_i8(xv[2u * gg], la, ia, 0, 0, 0);
+            ib = __builtin_amdgcn_mfma_i32_32x32x32_i8(xv[2u * gg], lb, ib, 0, 0, 0);
+            ia = __builtin_amdgcn_mfma_i32_32x32x32_i8(xv[2u * gg + 1u], ha, ia, 0, 0, 0);
+            ib = __builtin_amdgcn_mfma_i32_32x32x32_i8(xv[2u * gg + 1u], hb, ib, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            load_g(sn, gg);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        v16i isum;
+        // the row's mins as f16 pairs (64 m_j, m_j), j = 4 h .. 4 h + 3
+        v8h mb;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) isum[r] = (ia[r] << 3) + ib[r];
-        const float d = h2f_fast(mt.x & 0xFFFFu), dm = h2f_fast(mt.x >> 16);
+        for (uint32_t e = 0; e < 4u; ++e) {
+            const uint32_t mj = __builtin_amdgcn_ubfe(h ? mc.z : mc.y, 8u * e + 6u, 2) |
+                                (__builtin_amdgcn_ubfe(h ? mc.w >> 16 : mc.w, 4u * e, 4) << 2);
+            mb[2 * e] = (_Float16)(unsigned short)(mj << 6);
+            mb[2 * e + 1] = (_Float16)(unsigned short)mj;
+        }
+        const float d = h2f_fast(mc.x & 0xFFFFu), dm = h2f_fast(mc.x >> 16);
         {
-            const uint32_t ad = fb(dxl) & 0x7FFFFFFFu;            // the 32 tokens' scales, one a lane
+            const uint32_t ad = fb(dxl) & 0x7FFFFFFFu;             // the 32 tokens' scales, one a lane
             slow = slow || __ballot(ad != 0u && ad < 0x21800000u) != 0ull;   // wave-uniform, sticky
         }
+        v16f ms = {};
+        ms = __builtin_amdgcn_mfma_f32_32x32x16_f16(bs, mb, ms, 0, 0, 0);
         if (!slow) {
             // d Dx and dmin Dx as outer products on the matrix core (one IEEE product each; k = 1 is zero)
             v16f P1 = {}, P2 = {};
@@ -340,72 +395,93 @@ __global__ __launch_bounds__(512, GLU ? 2 : 4) void k_mm_q4k(MmArgs a) {
             P2 = __builtin_amdgcn_mfma_f32_32x32x2f32(dxl, h ? 0.0f : dm, P2, 0, 0, 0);
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const float tt = P1[r] * (float)isum[r] - P2[r] * ms[r];
+                const float tt = P1[r] * (float)((ia[r] << 3) + ib[r]) - P2[r] * ms[r];
                 p[r] = p[r] + tt;
             }
         } else {
-            // tokens of result r = 4 q + i: t0 + 8 q + 4 h + i
+            // tokens of result r = 4 q + e: t0 + 8 q + 4 h + e
             const float * xd = (const float *)(a.qa + a.d_off) + (size_t)a.tp * s + t0 + 4u * h;
-            float4 dx4[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) dx4[q] = *(const float4 *)(xd + 8u * q);
-            const float dxs[16] = { dx4[0].x, dx4[0].y, dx4[0].z, dx4[0].w, dx4[1].x, dx4[1].y, dx4[1].z, dx4[1].w,
-                                    dx4[2].x, dx4[2].y, dx4[2].z, dx4[2].w, dx4[3].x, dx4[3].y, dx4[3].z, dx4[3].w };
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const float tt = ssub(smul(smul(d, dxs[r]), i2f(isum[r])), smul(smul(dm, dxs[r]), ms[r]));
+                const float dx = xd[8 * (r >> 2) + (r & 3)];
+                const float tt = ssub(smul(smul(d, dx), i2f((ia[r] << 3) + ib[r])), smul(smul(dm, dx), ms[r]));
                 p[r] = sadd(p[r], tt);
             }
         }
+        __builtin_amdgcn_sched_barrier(0);
+        load_m(sn);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // fold the partial into the tree (the wave's own lanes in LDS): bit lv of pi set: it is the right half
+    // of level lv, else the left half, parked. The last partial has every bit set and stays in p.
+    bool open = true;
+#pragma unroll
+    for (int lv = 0; lv < kLev; ++lv) {
+        if (!open || (1u << lv) >= PG) continue;                   // wave-uniform
+        float4 (*sp)[64] = s_p[j][lv];
+        if ((pi >> lv) & 1u) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float4 u = sp[q][lane];
+                if (!slow) {
+                    p[4 * q] = u.x + p[4 * q]; p[4 * q + 1] = u.y + p[4 * q + 1];
+                    p[4 * q + 2] = u.z + p[4 * q + 2]; p[4 * q + 3] = u.w + p[4 * q + 3];
+                } else {
+                    p[4 * q] = sadd(u.x, p[4 * q]); p[4 * q + 1] = sadd(u.y, p[4 * q + 1]);
+                    p[4 * q + 2] = sadd(u.z, p[4 * q + 2]); p[4 * q + 3] = sadd(u.w, p[4 * q + 3]);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) sp[q][lane] = make_float4(p[4 * q], p[4 * q + 1], p[4 * q + 2], p[4 * q + 3]);
+            open = false;
+        }
+    }
     }
 #pragma unroll
-    for (int r = 0; r < 16; ++r) s_p[pj][64u * (uint32_t)r + lane] = p[r];
-    }
+    for (int q = 0; q < 4; ++q) s_p[j][0][q][lane] = make_float4(p[4 * q], p[4 * q + 1], p[4 * q + 2], p[4 * q + 3]);
     if (lane == 0u) s_slow[j] = slow ? 1 : 0;
-    lds_barrier();
-
-    bool any_slow = false;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) any_slow |= s_slow[i] != 0;
     uint32_t t64 = 0;
     if constexpr (GLU) t64 = a.ex.t64[lane];
-    // two outputs per thread, o = 64 r + lane of the wave layout above: weight row n0 + lane % 32,
-    // token t0 + 8 (r / 4) + 4 (lane / 32) + r % 4 (a wave stores 32 consecutive rows of 2 tokens)
-    for (uint32_t o = threadIdx.x; o < 1024u; o += 512u) {
-    const uint32_t ol = o & 63u, r = o >> 6;
-    const uint32_t nn = n0 + (ol & 31u), tt = t0 + 8u * (r >> 2) + 4u * (ol >> 5) + (r & 3u);
-    float v[16];
+    lds_barrier();
+
+    // wave j finishes the value quad q = j: weight row n0 + lane % 32, tokens t0 + 8 j + 4 (lane / 32) + e
+    const bool any_slow = (s_slow[0] | s_slow[1] | s_slow[2] | s_slow[3]) != 0;
+    const float4 u0 = s_p[0][0][j][lane], u1 = s_p[1][0][j][lane], u2 = s_p[2][0][j][lane], u3 = s_p[3][0][j][lane];
+    auto tree4 = [&](float w0, float w1, float w2, float w3) {
+        return canon(any_slow ? sadd(sadd(w0, w1), sadd(w2, w3)) : (w0 + w1) + (w2 + w3));
+    };
+    const float v[4] = { tree4(u0.x, u1.x, u2.x, u3.x), tree4(u0.y, u1.y, u2.y, u3.y), tree4(u0.z, u1.z, u2.z, u3.z),
+                         tree4(u0.w, u1.w, u2.w, u3.w) };
+    const uint32_t nn = n0 + c, t4 = t0 + 8u * j + 4u * h;
+    if constexpr (GLU) {
+        const bool odd = (lane & 1u) != 0u;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) v[i] = s_p[i][o];
-    if (!any_slow) {
-#pragma unroll
-        for (int w = 16; w > 1; w >>= 1)
-#pragma unroll
-            for (int i = 0; i < w / 2; ++i) v[i] = v[2 * i] + v[2 * i + 1];
+        for (int e = 0; e < 4; e += 2) {                           // every lane: the table is read by bpermute
+            const float a0 = dpp_f<kDppXor1>(v[e]), a1 = dpp_f<kDppXor1>(v[e + 1]);
+            const float hh = swiglu_reg(odd ? a1 : v[e], odd ? v[e + 1] : a0, a.ex, t64);
+            const uint32_t tt = t4 + (uint32_t)e + (odd ? 1u : 0u);
+            if (tt < a.T && nn < a.N) a.y[(size_t)tt * a.y_stride + (nn >> 1)] = hh;
+        }
     } else {
 #pragma unroll
-        for (int w = 16; w > 1; w >>= 1)
-#pragma unroll
-            for (int i = 0; i < w / 2; ++i) v[i] = sadd(v[2 * i], v[2 * i + 1]);
-    }
-    if constexpr (GLU) {
-        const float gt = canon(v[0]);
-        const float h = swiglu_reg(gt, dpp_f<kDppXor1>(gt), a.ex, t64);   // every lane: the table is read by bpermute
-        if ((ol & 1u) == 0u && tt < a.T && nn < a.N) a.y[(size_t)tt * a.y_stride + (nn >> 1)] = h;
-    } else if (tt < a.T && nn < a.N) {
-        float y = canon(v[0]);
-        float * yp = a.y + (size_t)tt * a.y_stride + nn;
-        if (a.add) y = sadd(a.add[(size_t)tt * a.add_stride + nn], y);
-        else if (a.acc) y = sadd(*yp, y);
-        *yp = y;
-    }
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t tt = t4 + (uint32_t)e;
+            if (tt < a.T && nn < a.N) {
+                float y = v[e];
+                float * yp = a.y + (size_t)tt * a.y_stride + nn;
+                if (a.add) y = sadd(a.add[(size_t)tt * a.add_stride + nn], y);
+                else if (a.acc) y = sadd(*yp, y);
+                *yp = y;
+            }
+        }
     }
 }
 
 }  // namespace tsr
 
 int tsr_launch_qact_mm4(const float * x, uint64_t x_stride, uint32_t K, uint32_t T, uint32_t tp, uint8_t * xq,
-                        int32_t * xs, float * xd, hipStream_t s) {
+                        uint32_t * xs, float * xd, hipStream_t s) {
     const uint64_t threads = (uint64_t)tp * (K / 256u) * 16u;
     if (threads + 255u >= 0x100000000ull) return -2;              // 32-bit pair indices
     hipLaunchKernelGGL(tsr::k_qact_mm4, dim3((uint32_t)((threads + 255u) / 256u)), dim3(256), 0, s, x, x_stride, K, T,
@@ -420,8 +496,8 @@ int tsr_launch_mm_q4_k(const tsr::MmArgs & a, hipStream_t s) {
     tsr::MmArgs m = a;
     m.grouped = (gx & 7u) == 0u && (uint64_t)a.N * (a.K / 256u) * 144u > (48ull << 20) ? 1u : 0u;   // measured
     const dim3 grid = m.grouped ? dim3(8u * gy, gx / 8u) : dim3(gx, gy);
-    if (a.glu) hipLaunchKernelGGL(tsr::k_mm_q4k<true>, grid, dim3(512), 0, s, m);
-    else hipLaunchKernelGGL(tsr::k_mm_q4k<false>, grid, dim3(512), 0, s, m);
+    if (a.glu) hipLaunchKernelGGL(tsr::k_mm_q4k<true>, grid, dim3(256), 0, s, m);
+    else hipLaunchKernelGGL(tsr::k_mm_q4k<false>, grid, dim3(256), 0, s, m);
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 

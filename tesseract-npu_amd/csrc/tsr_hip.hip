@@ -558,7 +558,7 @@ static int mul_mat_locked(tsr_hip_ctx * ctx, const tsr_hip_weight * w, const flo
         for (uint32_t t0 = 0; t0 < T; t0 += chunk) {
             const uint32_t tt = std::min(T - t0, chunk), tp = (tt + 31u) & ~31u;
             uint8_t * xq = (uint8_t *)ctx->scratch.ptr;
-            if (tsr_launch_qact_mm4(x_dev + (size_t)t0 * x_stride, x_stride, w->K, tt, tp, xq, (int32_t *)(xq + s_off),
+            if (tsr_launch_qact_mm4(x_dev + (size_t)t0 * x_stride, x_stride, w->K, tt, tp, xq, (uint32_t *)(xq + s_off),
                                     (float *)(xq + d_off), s))
                 return TSR_HIP_E_HIP;
             tsr::MmArgs m{};

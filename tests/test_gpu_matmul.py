@@ -191,3 +191,21 @@ def test_mm_q4_k_glu_llama_gate_up(dev, oc):
     assert_bits_equal(got, oc.swiglu(g, u), "GLU 8B gate|up")
     w.free()
     yb.free()
+
+
+@pytest.mark.parametrize("nsb", [1, 2, 3, 4, 5, 7, 8, 9, 12, 15, 16, 17, 23, 33])
+def test_mm_q4_k_partial_counts(dev, oc, nsb):
+    """Every way the 16 partials fall on the four waves of a tile (fewer super-blocks than waves, empty
+    partials, one or several super-blocks a partial), with token rows whose A256 scale is below 2^-60
+    (spec operations) beside ordinary ones, and with the largest integer sums: rows of equal values
+    (quants +-127, sub-block sums +-4064) against blocks of quant 15, scale and min 63."""
+    N, K, T = 40, 256 * nsb, 35
+    x = S.normal(900 + nsb, T * K).reshape(T, K)
+    x[3] *= np.float32(1e-22)
+    x[20], x[21] = 0.75, -0.75
+    x[22, ::2], x[22, 1::2] = 0.5, -0.5
+    blocks = weights(1, N, K, 70 + nsb).copy()
+    b = blocks.reshape(N, nsb, 144)
+    b[5, :, 4:] = 0xFF
+    got, want = _mm(dev, oc, N, K, T, x=x, wblocks=blocks, fmt=1)
+    assert_bits_equal(got, want, f"Q4_K {nsb} super-blocks")
