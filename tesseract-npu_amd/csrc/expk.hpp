@@ -58,7 +58,39 @@ __device__ __forceinline__ float expk_diff_with(float s, float m, float scale, c
 __device__ __forceinline__ float expk_diff(float s, float m, float scale, const ExpkTab & e, const uint32_t * t64) {
     return expk_diff_with(s, m, scale, e, [t64](uint32_t j) { return t64[j]; });
 }
-// The same with the table in a register: lane j of the wave holds t64[j] (read by ds_bpermute, no
+// EXPK(FM(FS(s, m), scale)) for s <= m in MAXT's order (every ASMAX exponent: m is the maximum, so the
+// argument v is <= 0 or NaN), in f64 arithmetic: EXPK's integers are products of up to 64 bits truncated to
+// integers, and with the f64 rounding mode set to truncation (f64_round_to_zero) fma(a, b, 2^52) holds
+// floor(a b) exactly in its low word. A step is a full-rate fma and add where the 32-bit form takes quarter-
+// rate integer products (~33 issue slots a value instead of ~60). v is cut off at -180, whose result is +0 as
+// that of everything below. Equal to the restatement of the reference on all 2^31 negative floats (a CPU
+// run in the truncating mode). td: t64[j] 2^-32 as f64, in LDS.
+// The wave's f64 (and f16) operations truncate from here on (MODE.FP_ROUND[3:2] = toward zero); f32 keeps
+// rounding to nearest even. In asm, because the compiler takes a mode set by its builtin back in front of
+// the next f64 operation. x: a value on which every f64 operation meant depends (the only order that the
+// compiler keeps between them and the asm).
+__device__ __forceinline__ void f64_round_to_zero(float & x) {
+    asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 3\n\ts_nop 7" : "+v"(x));
+}
+__device__ __forceinline__ float expk_neg_diff(float s, float m, float scale, const ExpkNeg & e, const double * td) {
+    constexpr double k52 = 4503599627370496.0;
+    const float d = s - m;
+    const float dz = __builtin_amdgcn_classf(d, 0x90) ? bf(fb(d) & 0x80000000u) : d;
+    const float v = dz * scale;
+    const double T = __builtin_fma((double)__builtin_fmaxf(v, -180.0f), -e.lk, k52);   // 2^52 + |v| log2(e) 2^32
+    const uint64_t r = __builtin_bit_cast(uint64_t, (9007199254740992.0 + 2251799813685248.0) - T);   // 2^52 + 2^51 - T
+    const uint32_t F = (uint32_t)r;
+    const double G = __builtin_bit_cast(double, 0x4130000000000000ull | (F & 0x03FFFFFFu)) - 1048576.0;   // G 2^-32
+    const double m1 = __builtin_fma(G, e.c3, k52);
+    const double m2 = __builtin_fma(G, m1 + e.c2, k52);
+    const double m3 = __builtin_fma(G, m2 + e.c1, k52);
+    const double M = __builtin_fma(td[F >> 26], m3 + (4294967296.0 - k52), k52);
+    const uint32_t fm = fb((float)(uint32_t)__builtin_bit_cast(uint64_t, M));
+    const uint32_t x = fm + (((uint32_t)(r >> 32) - (0x43380000u + 30u)) << 23);   // the exponent moved by n0 - 30
+    const uint32_t q = (int32_t)x < 0x00800000 ? 0u : x;
+    return bf(v != v ? kNaN : q);
+}
+// EXPK with the table in a register: lane j of the wave holds t64[j] (read by ds_bpermute, no
 // LDS table and no barrier).
 __device__ __forceinline__ float expk_reg(float v, const ExpkTab & e, uint32_t t64_lane) {
     return expk_with(v, e, [t64_lane](uint32_t j) {

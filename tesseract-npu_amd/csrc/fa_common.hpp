@@ -86,11 +86,13 @@ __device__ __forceinline__ float bf_scale(float f, int32_t k) {
 
 typedef int v4i_fa __attribute__((ext_vector_type(4)));
 
-// A = d0 + 256 d1 + 65536 d2 + 2^24 d3 of four digit sums (|d_k| <= 2^20): every product and partial
-// sum is exact in f64 (|A| < 2^45), and the one conversion to f32 is RNE24(A).
+// RNE24(A) of A = d0 + 256 d1 + 65536 d2 + 2^24 d3, four digit sums (|d_k| <= 2^20, so |A| < 2^45): the
+// pairs are exact in int32 (< 2^29), and A = hi 2^23 + lo with lo in [0, 2^23) and |hi| < 2^22, both exact in
+// f32, is rounded once by the fma. (In f64, four conversions and six operations, it was the longest part
+// of the P.V product's output.)
 __device__ __forceinline__ float digits_rne24(const v4i_fa & acc) {
-    const double A = ((double)acc[3] * 16777216.0 + (double)acc[2] * 65536.0) + ((double)acc[1] * 256.0 + (double)acc[0]);
-    return (float)A;
+    const int32_t l = acc[0] + (acc[1] << 8), h = acc[2] + (acc[3] << 8) + (l >> 16);   // A = h 2^16 + (l & 0xFFFF)
+    return __builtin_fmaf((float)(h >> 7), 8388608.0f, (float)(((h & 127) << 16) | (l & 0xFFFF)));
 }
 
 // Data that blocks on other XCDs read after a counter moves only through accesses coherent at agent

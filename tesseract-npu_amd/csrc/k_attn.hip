@@ -123,40 +123,105 @@ struct PvBlock {
         for (uint32_t t8 = 0; t8 < 2 * BB; ++t8) L.bq[t8] = *(const int4 *)(vqB + 256u * t8);
     }
 
+    // The digits of the weights' integers W = RNE_int(w 2^(23 - es)) of the lane's 4 cells to LDS, for block e
+    // and digit k in one word; the fences keep the wave's own LDS accesses in order.
+    __device__ __forceinline__ void digits(const float (&w)[4][BB], int32_t es, uint8_t * dg) const {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (uint32_t e = 0; e < BB; ++e) {
+            uint32_t P[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) P[i] = ((uint32_t)bf_int_n(w[i][e], es) + 0x80808080u) ^ 0x80808080u;   // byte k = digit k
+            // transpose the 4 x 4 bytes: word k = digit k of cells 0..3
+            const uint32_t lo01 = __builtin_amdgcn_perm(P[1], P[0], 0x05010400u);   // d0c0 d0c1 d1c0 d1c1
+            const uint32_t lo23 = __builtin_amdgcn_perm(P[3], P[2], 0x05010400u);
+            const uint32_t hi01 = __builtin_amdgcn_perm(P[1], P[0], 0x07030602u);   // d2c0 d2c1 d3c0 d3c1
+            const uint32_t hi23 = __builtin_amdgcn_perm(P[3], P[2], 0x07030602u);
+            const uint32_t q[4] = { __builtin_amdgcn_perm(lo23, lo01, 0x05040100u), __builtin_amdgcn_perm(lo23, lo01, 0x07060302u),
+                                    __builtin_amdgcn_perm(hi23, hi01, 0x05040100u), __builtin_amdgcn_perm(hi23, hi01, 0x07060302u) };
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                *(uint32_t *)(dg + (((e * 4u + hr) * 4u + (uint32_t)k) * 4u + kk) * 16u + 4u * quad) = q[k];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+
     // One segment (L holds its loads): EXP, LSUM, the block-float weights, their digits and the
     // matrix-core digit sums; the segment's results go to s_c [slot][4 heads][DV] and s_l [slot][4 heads].
-    __device__ __forceinline__ void segment(uint32_t seg, uint32_t slot, Loads & L, float m, const uint32_t * s_t64,
-                                            float * s_c, float * s_l, uint8_t * dg) const {
+    // The common case of a batch (wave-uniform: every p and value scale finite, every head row's largest
+    // weight 0 or in [2^-102, 2^106)) needs no flag and no flush: with the segment exponent E_S >= -102 a
+    // subnormal weight rounds to W = 0 as the flushed one does, and with |A| in [1, 2^45) the scaled result
+    // is a normal number for E_S in -102 .. 105. The general form runs otherwise.
+    // Returns whether every batch was the common case.
+    __device__ __forceinline__ bool segment(uint32_t seg, uint32_t slot, Loads & L, float m, const ExpkNeg & en,
+                                            const double * s_td, float * s_c, float * s_l, uint8_t * dg) const {
+        bool common = true;
         // ---- phase A: lane = (head row, 4 cells) ----------------------------------------------
         const bool cv = 4u * seg + kk < nu;
         const float ss[4] = { L.sv.x, L.sv.y, L.sv.z, L.sv.w };
         float pz[4];
-        uint32_t pnf = 0u, pe = 0u;                                // non-finite flag; largest exponent field
+        uint32_t pm = 0u;                                          // largest p (not negative; NaN above all)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            // EXPK results are zero, normal, Inf or NaN (never subnormal)
-            const float ez = expk_diff(ss[i], m, a.scale, a.ex, s_t64);   // straight-line, then the select
+            // EXPK results are zero, normal or NaN (never subnormal)
+            const float ez = expk_neg_diff(ss[i], m, a.scale, en, s_td);   // straight-line, then the select
             pz[i] = (cv && head_ok) ? ez : 0.0f;
-            const uint32_t f = f_field(pz[i]);
-            pnf |= f == 255u ? 1u : 0u;
-            pe = max(pe, f == 255u ? 0u : f);
+            pm = max(pm, fb(pz[i]));
         }
-        // LSUM of the segment (AT 6.5): block float of its p values
+        const bool pfin = __ballot(pm >= 0x7F800000u) == 0ull;
+        // LSUM of the segment (AT 6.5): block float of its p values; NaN when one is (EXPK of a value <= 0 is
+        // at most 1, so a p that is not finite is NaN)
         if (vh == 0u) {
-            const bool badl = row16_or(pnf) != 0u;
-            pe = row16_umax(pe);
+            pm = row16_umax(pm);
+            const int32_t pe = (int32_t)(pm >> 23);                // the largest exponent field (255: the sum is not used)
             int32_t lsum = 0;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) lsum += f_field(pz[i]) == 255u ? 0 : bf_int_n(pz[i], (int32_t)pe - 127);
+            for (int i = 0; i < 4; ++i) lsum += bf_int_n(pm >= 0x7F800000u ? 0.0f : pz[i], pe - 127);
             lsum = row16_isum(lsum);
             if ((lane & 15u) == 0u)
-                s_l[slot * 4u + hr] = badl ? bf(kNaN) : (pe == 0u ? 0.0f : bf_scale((float)lsum, (int32_t)pe - 150));
+                s_l[slot * 4u + hr] = pe == 255 ? bf(kNaN) : (pe == 0 ? 0.0f : bf_scale((float)lsum, pe - 150));
         }
 
 #pragma unroll
         for (uint32_t bt = 0; bt < NBT; ++bt) {                    // BB value blocks (32 BB values) at a time
             const uint32_t vb = vb0 + bt * BB;
             if (bt > 0u) loads(seg, vb, L, false);
+            static_assert(BB == 2, "one 64-value slice a batch");
+            const uint32_t chk = ((L.mb[0][0] & 0x7C007C00u) + 0x04000400u) | ((L.mb[0][1] & 0x7C007C00u) + 0x04000400u) |
+                                 ((L.mb[1][0] & 0x7C007C00u) + 0x04000400u) | ((L.mb[1][1] & 0x7C007C00u) + 0x04000400u);
+            float wf[4][BB], mx = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+#pragma unroll
+                for (uint32_t e = 0; e < BB; ++e)
+                    wf[i][e] = pz[i] * h2f_fast((L.mb[e][i >> 1] >> (16u * (i & 1u))) & 0xFFFFu);
+                mx = __builtin_fmaxf(mx, __builtin_fmaxf(__builtin_fabsf(wf[i][0]), __builtin_fabsf(wf[i][1])));
+            }
+            const uint32_t mr = row16_umax(fb(mx));                // largest |w| of the head row (not negative)
+            const int32_t ef = (int32_t)(mr >> 23) - 127;
+            const bool okf = pfin && (chk & 0x80008000u) == 0u && (mr == 0u || (ef >= -102 && ef <= 105));
+            if (__builtin_expect(__ballot(!okf) == 0ull, 1)) {
+                digits(wf, ef, dg);
+#pragma unroll
+                for (uint32_t e = 0; e < BB; ++e) {
+                    const v4i_fa Aop = *(const v4i_fa *)(dg + ((e * 16u + (lane & 15u)) * 4u + (lane >> 4)) * 16u);
+#pragma unroll
+                    for (int half = 0; half < 2; ++half) {
+                        const int4 bq = L.bq[2 * e + half];
+                        const v4i_fa Bop = { bq.x, bq.y, bq.z, bq.w };
+                        v4i_fa acc = { 0, 0, 0, 0 };
+                        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop, Bop, acc, 0, 0, 0);
+                        s_c[(slot * 4u + hr) * DV + 32u * (bt * BB + e) + 16u * (uint32_t)half + (lane & 15u)] =
+                            __builtin_ldexpf(digits_rne24(acc), ef - 23);
+                    }
+                }
+                continue;
+            }
+            common = false;
             // weights of the 4 cells for the BB blocks: w = p dV, a subnormal product flushed to zero
             float w[4][BB];
             uint32_t ex[BB / 2], nfm = 0u;
@@ -184,33 +249,13 @@ struct PvBlock {
                 es[sa] = (int32_t)ef - 127;
             }
             const uint32_t badm = row16_or(nfm);
-            // digits: for block e and digit k, the 4 cells' digit bytes in one word
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-            for (uint32_t e = 0; e < BB; ++e) {
-                const bool use = any[e >> 1] && ((badm >> e) & 1u) == 0u;
-                uint32_t P[4];
+            for (uint32_t e = 0; e < BB; ++e)
+                if (!any[e >> 1] || ((badm >> e) & 1u) != 0u) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int32_t W = use ? bf_int_n(w[i][e], es[e >> 1]) : 0;
-                    P[i] = ((uint32_t)W + 0x80808080u) ^ 0x80808080u;     // byte k = digit k of W
+                    for (int i = 0; i < 4; ++i) w[i][e] = 0.0f;
                 }
-                // transpose the 4 x 4 bytes: word k = digit k of cells 0..3
-                const uint32_t lo01 = __builtin_amdgcn_perm(P[1], P[0], 0x05010400u);   // d0c0 d0c1 d1c0 d1c1
-                const uint32_t lo23 = __builtin_amdgcn_perm(P[3], P[2], 0x05010400u);
-                const uint32_t hi01 = __builtin_amdgcn_perm(P[1], P[0], 0x07030602u);   // d2c0 d2c1 d3c0 d3c1
-                const uint32_t hi23 = __builtin_amdgcn_perm(P[3], P[2], 0x07030602u);
-                const uint32_t q[4] = { __builtin_amdgcn_perm(lo23, lo01, 0x05040100u), __builtin_amdgcn_perm(lo23, lo01, 0x07060302u),
-                                        __builtin_amdgcn_perm(hi23, hi01, 0x05040100u), __builtin_amdgcn_perm(hi23, hi01, 0x07060302u) };
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    *(uint32_t *)(dg + (((e * 4u + hr) * 4u + (uint32_t)k) * 4u + kk) * 16u + 4u * quad) = q[k];
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            digits(w, es[0], dg);
             // ---- phase B: 2 BB tiles of 16 values; lane = (head row l / 16 of the result, value l % 16)
 #pragma unroll
             for (uint32_t e = 0; e < BB; ++e) {
@@ -228,18 +273,26 @@ struct PvBlock {
                 }
             }
         }
+        return common;
     }
 
     // After a block barrier: the segment chains in order (AT 6.4 O, 6.5 l) -> the channel partials.
-    // Thread = (head row, value of the part).
-    __device__ __forceinline__ void chains(uint32_t item, uint32_t hg, const float * s_c, const float * s_l) const {
+    // Thread = (head row, value of the part). common: every batch of every segment was the common case, so
+    // every result is a multiple of 2^(E_S - 23) >= 2^-125, and so is every rounded sum of them: none is
+    // subnormal, and the chain needs no FTZ.
+    __device__ __forceinline__ void chains(uint32_t item, uint32_t hg, const float * s_c, const float * s_l,
+                                           bool common) const {
         const uint32_t G = a.G, nh = a.n_head;
         for (uint32_t idx = threadIdx.x; idx < 4u * DV; idx += blockDim.x) {
             const uint32_t r4 = idx / DV, v = idx % DV, hi2 = 4u * hg + r4;
             if (hi2 >= G) continue;
             const uint32_t h2 = g * G + hi2;
             float O = 0.0f;
-            for (uint32_t seg = 0; seg < nseg; ++seg) O = sadd_z(O, s_c[(seg * 4u + r4) * DV + v]);
+            if (__builtin_expect(common, 1)) {
+                for (uint32_t seg = 0; seg < nseg; ++seg) O = O + s_c[(seg * 4u + r4) * DV + v];
+            } else {
+                for (uint32_t seg = 0; seg < nseg; ++seg) O = sadd_z(O, s_c[(seg * 4u + r4) * DV + v]);
+            }
             const size_t slot = ((size_t)item * 4u + c) * nh + h2;
             a.OP[slot * D + vh * DV + v] = canon(O);
             if (vh == 0u && v == 0u) {
@@ -453,6 +506,176 @@ __global__ __launch_bounds__(256) void k_fa_qk(FaArgs a, FaPlan p) {
     }
 }
 
+// ---------------------------------------------------------------------------------------------
+// scores of many rows on the matrix cores: block (256-cell tile, 32 rows, query head), 4 waves of two 32-cell
+// subtiles. The rows' runs start at one cell, so their chunk cuts are multiples of 16 groups from there and
+// every row's 256-cell tiles are the same cells; the item of each (tile, row) comes from the host's map.
+//
+// Per 32 rows x 32 cells and 32-value block, as in the prefill MUL_MAT: the integer block sums are one
+// v_mfma_i32_32x32x32_i8 (rows: queries, columns: cells) and the products dK Dx one
+// v_mfma_f32_32x32x2f32 with a zero second column; the score is the block terms' tree. A lane holds one
+// cell of 16 rows, so 32 lanes store 32 consecutive scores of a row. While every scale of the wave is finite
+// no score is Inf or NaN: the canonicalization and the NaN rule of the maximum are left to waves that met
+// one (sticky). The rows' store offsets are read from LDS where they are needed: with them in registers the
+// kernel spilled, and a reload waits for the stores in front of it (the memory counter retires in order).
+//
+// The one-row kernel below reads each K row per query row and spends ~130 VALU operations a score; this one
+// ~20.
+// ---------------------------------------------------------------------------------------------
+typedef float v16f_fa __attribute__((ext_vector_type(16)));
+typedef int v16i_fa __attribute__((ext_vector_type(16)));
+
+template <int D>
+__global__ __launch_bounds__(256, 3) void k_fa_qk_mm(FaArgs a, uint32_t T) {
+    constexpr uint32_t NBD = D / 32u;
+    __shared__ uint32_t s_hi[32], s_end[32], s_tile[32];           // of the block's rows: run end, item end, Mpart row
+    __shared__ __align__(16) uint32_t s_vo[32];                    // byte offset of the row's score of the tile's first cell
+    __shared__ __align__(16) float s_mx[4][64][20];                // each wave's maxima of the lane's 16 rows (padded)
+    const uint32_t at = blockIdx.x, t0 = 32u * blockIdx.y, h = blockIdx.z, g = h / a.G;
+    const uint32_t lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t c = lane & 31u, hh = lane >> 5;
+    const uint32_t cell0 = 16u * (a.u_lo + 16u * at);              // first cell of the tile
+    const uint32_t ng = (a.kc.kv_size + 15u) / 16u, E = a.E, nbk = E / 32u;
+    // this wave's first K operands and its query operands: they depend on no item
+    const uint32_t t = min(t0 + c, T - 1u);
+    v4i_fa kr[NBD], xv[NBD];
+    uint32_t km[NBD];
+    float dx[NBD];
+    auto load_k = [&](uint32_t sub) {                              // clamped: loads stay inside the plane
+        const uint32_t u0 = min((cell0 + 32u * sub) >> 4, ng - 1u), u = min(u0 + (c >> 4), ng - 1u) - u0;
+        const uint8_t * kq = a.kc.base + a.kc.quant_off + ((size_t)u0 * E + (size_t)g * D) * 16u;
+        const uint8_t * kmeta = a.kc.base + ((size_t)u0 * nbk + (size_t)g * NBD) * 32u;
+        const uint32_t oq = u * 16u * E + hh * 256u + (c & 15u) * 16u, om = (u * nbk * 16u + (c & 15u)) * 2u;
+#pragma unroll
+        for (uint32_t b = 0; b < NBD; ++b) {
+            kr[b] = *(const v4i_fa *)(kq + (oq + 512u * b));
+            km[b] = *(const uint16_t *)(kmeta + (om + 32u * b));
+        }
+    };
+#pragma unroll
+    for (uint32_t b = 0; b < NBD; ++b) {                           // block b at xq + ((h NBD + b) T + t) 32
+        const uint32_t o = (h * NBD + b) * T + t;
+        xv[b] = *(const v4i_fa *)(a.xq + (size_t)o * 32u + 16u * hh);
+        dx[b] = a.xd[o];
+    }
+    load_k(2u * wave);
+    __builtin_amdgcn_sched_barrier(0);
+    // the rows' items (every wave reads them; wave 0 publishes)
+    const uint32_t idx = t0 + c < T ? a.tmap[(size_t)at * T + t] : 0xFFFFFFFFu;
+    uint32_t end = 0u, hi = 0u;
+    if (idx != 0xFFFFFFFFu) {
+        const FaItem it = a.items[idx];
+        const uint32_t c0 = 16u * it.u0, n16 = 16u * it.n;
+        end = c0 + n16;
+        hi = a.hi[t];                                              // a run ends inside its last item
+        if (threadIdx.x < 32u) {
+            s_vo[c] = 4u * (it.s_off * a.n_head + h * n16 + (cell0 - c0));
+            s_tile[c] = it.tile0 + (cell0 - c0) / 256u;
+        }
+    }
+    if (threadIdx.x < 32u) {
+        s_hi[c] = hi;
+        s_end[c] = end;
+    }
+    uint32_t top = end, all = hi;       // the last item end of the rows; the cells below `all` are visible to every row
+#pragma unroll
+    for (int sh = 16; sh >= 1; sh >>= 1) {
+        top = max(top, (uint32_t)shfl_i((int)top, (int)(lane ^ (uint32_t)sh)));
+        all = min(all, (uint32_t)shfl_i((int)all, (int)(lane ^ (uint32_t)sh)));
+    }
+    top = __builtin_amdgcn_readfirstlane(top);
+    all = __builtin_amdgcn_readfirstlane(all);
+    if (top <= cell0) return;                                      // no row reaches the tile (block-uniform)
+    lds_barrier();
+
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(a.S, 0, (int)a.s_bytes, 0x00020000);
+    const float ninf = bf(kNegInf);
+    bool fin = true;
+    float mx[16];
+#pragma unroll
+    for (uint32_t b = 0; b < NBD; ++b) {
+        fin = fin && !__builtin_amdgcn_classf(dx[b], 0x207);
+        dx[b] = hh ? 0.0f : dx[b];                                 // the k = 1 column of the scale product
+    }
+#pragma unroll
+    for (uint32_t r = 0; r < 16u; ++r) mx[r] = bf(kMFloor);
+    bool slow = __ballot(!fin) != 0ull;
+#pragma unroll
+    for (uint32_t k2 = 0; k2 < 2u; ++k2) {
+        const uint32_t sub = 2u * wave + k2, cs = cell0 + 32u * sub;
+        bool kfin = true;
+        v16f_fa s[NBD / 2u];                                       // the tree's first level
+#pragma unroll
+        for (uint32_t b = 0; b < NBD; ++b) {
+            v16i_fa is = {};
+            is = __builtin_amdgcn_mfma_i32_32x32x32_i8(xv[b], kr[b], is, 0, 0, 0);
+            kfin = kfin && (km[b] & 0x7C00u) != 0x7C00u;
+            v16f_fa P = {};
+            P = __builtin_amdgcn_mfma_f32_32x32x2f32(dx[b], hh ? 0.0f : h2f_fast(km[b]), P, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float p = P[r] * (float)is[r];
+                if (b & 1u) s[b >> 1][r] = s[b >> 1][r] + p;
+                else s[b >> 1][r] = p;
+            }
+            __builtin_amdgcn_sched_barrier(0);                     // one block's products in registers at a time
+        }
+        slow = slow || __ballot(!kfin) != 0ull;
+#pragma unroll
+        for (uint32_t w = NBD / 4u; w >= 1u; w >>= 1)
+#pragma unroll
+            for (uint32_t k = 0; k < w; ++k)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[k][r] = s[2u * k][r] + s[2u * k + 1u][r];
+        __builtin_amdgcn_sched_barrier(0);
+        if (k2 == 0u) load_k(sub + 1u);                            // ahead of the stores (the counter retires in order)
+        __builtin_amdgcn_sched_barrier(0);
+        // +0 once (see k_fa_qk); cells outside a row's run are -inf, outside its item not stored
+        const uint32_t vc = 128u * sub + 4u * c;
+        if (!slow && cs >= a.lo && cs + 32u <= all) {              // wave-uniform: every cell visible to every row
+#pragma unroll
+            for (uint32_t q = 0; q < 4u; ++q) {
+                const uint4 vo = *(const uint4 *)&s_vo[8u * q + 4u * hh];
+#pragma unroll
+                for (uint32_t e = 0; e < 4u; ++e) {
+                    const float v = s[0][4u * q + e] + 0.0f;
+                    const uint32_t o = e == 0u ? vo.x : (e == 1u ? vo.y : (e == 2u ? vo.z : vo.w));
+                    __builtin_amdgcn_raw_buffer_store_b32(fb(v), rs, (int)(o + vc), 0, 0);
+                    mx[4u * q + e] = __builtin_fmaxf(mx[4u * q + e], v);
+                }
+            }
+        } else {
+#pragma unroll
+            for (uint32_t r = 0; r < 16u; ++r) {
+                const uint32_t row = 8u * (r >> 2) + 4u * hh + (r & 3u), cell = cs + c;
+                const float x = canon(s[0][r] + 0.0f);
+                const float v = cell >= a.lo && cell < s_hi[row] ? x : ninf;
+                const bool in = cell < s_end[row];
+                if (in) __builtin_amdgcn_raw_buffer_store_b32(fb(v), rs, (int)(s_vo[row] + vc), 0, 0);
+                const float w = in ? v : bf(kMFloor);
+                mx[r] = slow ? maxt(mx[r], w) : __builtin_fmaxf(mx[r], w);
+            }
+        }
+    }
+    // the rows' maxima over the tile: value r of lane l is row 8 (r / 4) + 4 (l / 32) + r % 4
+#pragma unroll
+    for (uint32_t q = 0; q < 4u; ++q)
+        *(float4 *)&s_mx[wave][lane][4u * q] = make_float4(mx[4u * q], mx[4u * q + 1u], mx[4u * q + 2u], mx[4u * q + 3u]);
+    lds_barrier();
+    {
+        const uint32_t row = threadIdx.x >> 3, l8 = threadIdx.x & 7u, r = 4u * (row >> 3) + (row & 3u), half = (row >> 2) & 1u;
+        uint32_t k = 0u;
+#pragma unroll
+        for (uint32_t w = 0; w < 4u; ++w)
+#pragma unroll
+            for (uint32_t e = 0; e < 4u; ++e) k = umax_u(k, maxt_key_f(s_mx[w][32u * half + 8u * e + l8][r]));
+        k = umax_u(k, (uint32_t)dpp_i<kDppXor1>((int)k));
+        k = umax_u(k, (uint32_t)dpp_i<kDppXor2>((int)k));
+        k = umax_u(k, (uint32_t)dpp_i<kDppRowHalfMirror>((int)k));
+        if (l8 == 0u && s_end[row] > cell0) a.Mpart[(size_t)s_tile[row] * a.n_head + h] = maxt_unkey(k);
+    }
+}
+
 template <int D, bool INL, int VS>
 __global__ __launch_bounds__(64 * kPvWaves) void k_fa_pv(FaArgs a, FaPlan p) {
     extern __shared__ __align__(16) uint8_t lds[];
@@ -462,8 +685,8 @@ __global__ __launch_bounds__(64 * kPvWaves) void k_fa_pv(FaArgs a, FaPlan p) {
     // the launch has one wave per segment of its longest channel (nw <= kPvWaves), so the segment
     // results need nw slots: the LDS is sized by the launch
     const uint32_t nw = blockDim.x >> 6;
-    uint32_t * s_t64 = (uint32_t *)lds;                           // EXPK table
-    float * s_c = (float *)(lds + 256);                           // [seg][4 heads][DV]
+    double * s_td = (double *)lds;                                // EXPK table
+    float * s_c = (float *)(lds + 512);                           // [seg][4 heads][DV]
     float * s_l = s_c + nw * 4u * DV;                             // [seg][4 heads]
     uint8_t * s_dg = (uint8_t *)(s_l + nw * 4u);                  // per wave: [BB blocks][4 heads][4 digits][4 groups][16]
     const uint32_t t64v = a.ex.t64[threadIdx.x & 63u];            // first: the table write waits for it only
@@ -479,17 +702,19 @@ __global__ __launch_bounds__(64 * kPvWaves) void k_fa_pv(FaArgs a, FaPlan p) {
     typename PB::Loads L;
     if (wave < pb.nseg) pb.loads(wave, pb.vb0, L, true);
     __builtin_amdgcn_sched_barrier(0);
-    if (threadIdx.x < 64u) s_t64[threadIdx.x] = t64v;
+    if (threadIdx.x < 64u) s_td[threadIdx.x] = (double)t64v * 0x1p-32;
+    const ExpkNeg & en = a.en;
     lds_barrier();
 
     // chunk maximum of head h: MAXOUT of the floor and the tile maxima (row lanes < ntiles read one each)
-    const float m = maxt_unkey(row16_umax(max(mkey, maxt_key_f(bf(kMFloor)))));
+    float m = maxt_unkey(row16_umax(max(mkey, maxt_key_f(bf(kMFloor)))));
+    f64_round_to_zero(m);
+    bool common = true;
     for (uint32_t seg = wave; seg < pb.nseg; seg += nw) {
         if (seg != wave) pb.loads(seg, pb.vb0, L, true);
-        pb.segment(seg, seg, L, m, s_t64, s_c, s_l, dg);
+        common = pb.segment(seg, seg, L, m, en, s_td, s_c, s_l, dg) && common;
     }
-    __syncthreads();
-    pb.chains(item, hg, s_c, s_l);
+    pb.chains(item, hg, s_c, s_l, __syncthreads_and(common) != 0);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -618,7 +843,14 @@ static int launch_fa(const tsr::FaArgs & a, const tsr::FaPlan & p, uint32_t T, u
     const bool rope = a.cell != nullptr;                          // ROPE + SET_ROWS_KV fused (host-checked shape)
     const size_t lds_qk = tsr::fa_qk_lds(a.G, a.D, rope);
     const dim3 gqk(p.n_items * p.maxtiles, a.n_head_kv);
-    if (rope) {
+    if (a.tmap != nullptr) {                                      // many rows: scores on the matrix cores (host-checked)
+        const dim3 gmm(a.n_map, (T + 31u) / 32u, a.n_head), bmm(256);
+        switch (a.D) {
+            case 64: hipLaunchKernelGGL(tsr::k_fa_qk_mm<64>, gmm, bmm, 0, s, a, T); break;
+            case 128: hipLaunchKernelGGL(tsr::k_fa_qk_mm<128>, gmm, bmm, 0, s, a, T); break;
+            default: return -2;
+        }
+    } else if (rope) {
         switch (a.D) {
             case 64: hipLaunchKernelGGL((tsr::k_fa_qk<64, INL, true>), gqk, dim3(256), lds_qk, s, a, p); break;
             case 128: hipLaunchKernelGGL((tsr::k_fa_qk<128, INL, true>), gqk, dim3(256), lds_qk, s, a, p); break;
@@ -647,7 +879,7 @@ static int launch_fa(const tsr::FaArgs & a, const tsr::FaPlan & p, uint32_t T, u
     uint32_t vs = 1;
     while (vs < 4u && a.D / (2u * vs) >= 64u && blocks * vs < 2ull * n_cu) vs *= 2u;
     const uint32_t dv = a.D / vs, bb = 2u;                        // PvBlock::BB
-    const size_t lds_pv = 256u + 4u * (size_t)nwv * 4u * dv + 4u * nwv * 4u + 1024u * bb * nwv;
+    const size_t lds_pv = 512u + 4u * (size_t)nwv * 4u * dv + 4u * nwv * 4u + 1024u * bb * nwv;
     const dim3 gpv(4u * p.n_items, a.n_head_kv, (a.G + 3u) / 4u * vs);
     const dim3 bpv(64u * nwv);
 #define TSR_PV(DD, VV) hipLaunchKernelGGL((tsr::k_fa_pv<DD, INL, VV>), gpv, bpv, lds_pv, s, a, p)

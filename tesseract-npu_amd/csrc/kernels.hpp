@@ -23,6 +23,12 @@ struct ExpkTab {
     uint64_t lk, c1, c2, c3;
 };
 
+// The same constants for EXPK of arguments <= 0 in f64 (expk.hpp: expk_neg_diff): LK 2^-6, c3, c2 - 2^52,
+// c1 - 2^52.
+struct ExpkNeg {
+    double lk, c3, c2, c1;
+};
+
 // What the matvec applies to x in front of its activation quantization (MvArgs::prep).
 enum MvPrep : uint32_t {
     kPrepNone = 0,           // x as given
@@ -129,6 +135,15 @@ struct FaArgs {
     uint32_t n_dims, neox;
     float ts, m;
     const float * rtab;      // or the angles of *pos from tsr_hip_rope_table: [n_dims / 2] (M cos, M sin)
+    // the scores of many rows on the matrix cores (k_fa_qk_mm; tmap != 0): the query rows quantized by
+    // k_qact_mm at xq / xd, and the item of every (256-cell tile from group u_lo on, row): [n_map][T], ~0u none
+    ExpkNeg en;
+    const uint32_t * tmap;
+    const uint8_t * xq;
+    const float * xd;
+    uint32_t n_map, u_lo, lo;  // lo: the first visible cell of every row (the runs' common start)
+    const uint32_t * hi;     // [T] the end of each row's run
+    uint32_t s_bytes;        // bytes of S
 };
 
 // The one-launch decode FLASH_ATTN_EXT (k_fa_dec.hip): one query row over a plan's device work list,

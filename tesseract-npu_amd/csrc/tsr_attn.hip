@@ -421,6 +421,7 @@ tsr::FaArgs fa_args(tsr_hip_ctx * ctx, const float * q_dev, uint64_t q_stride, c
     a.out = out_dev;
     a.out_stride = out_stride;
     a.ex = ctx->expk;
+    a.en = { (double)a.ex.lk * 0x1p-6, (double)a.ex.c3, (double)a.ex.c2 - 0x1p52, (double)a.ex.c1 - 0x1p52 };   // exact
     return a;
 }
 
@@ -453,8 +454,29 @@ static int fa_unplanned(tsr_hip_ctx * ctx, const float * q_dev, uint32_t T, uint
     if (w.cells * n_head > 0xFFFFFFFFull || n_items * 4u > 0x7FFFFFFFull || n_items * w.maxtiles > 0x7FFFFFFFull)
         return TSR_HIP_E_SHAPE;
     const bool inl = n_items <= tsr::kFaInlItems && T <= tsr::kFaInlTok;
+    // The scores of many rows on the matrix cores (k_fa_qk_mm): one FAST run per row, all from one cell, so
+    // that the rows' chunk cuts (multiples of 16 groups) fall on common 256-cell tiles. It needs the queries'
+    // quantization as a launch of its own (3-6 us), and pays from ~4 M scores of D 128 on. Measured, one-row
+    // kernel -> QACT + this one: 512 rows behind 1536 cells (29 M scores) 110 -> 56 us, 300 rows behind 700
+    // (8 M) 38 -> 30, D 64: 256 rows from cell 0 (1.3 M) 9.4 -> 13.7.
+    uint32_t n_map = 0, lo = 0;
+    if constexpr (!NOALLOC) {
+        bool uni = !inl && D <= 128u && (msum[3] & 1u) == 0u && w.cells * n_head * (D / 64u) >= (10ull << 20) &&
+                   4u * w.cells * n_head < (1ull << 31) && (uint64_t)T * K < (1ull << 31);
+        lo = msum[8];
+        for (uint32_t t = 0; uni && t < T; ++t) {
+            const uint32_t * r = msum + 8u + 4u * t;
+            uni = r[0] == lo && r[1] > r[0] && r[2] >= r[3];
+            n_map = std::max(n_map, ((r[1] + 15u) / 16u - lo / 16u + 15u) / 16u);
+        }
+        if (!uni) n_map = 0;
+    }
     size_t off = 0;
-    const size_t o_items = off; off = up256(off + (inl ? 0u : n_items * sizeof(tsr::FaItem) + 8u * (size_t)T));
+    const size_t map_words = n_map ? (size_t)n_map * T + T : 0u;  // the tile map and the rows' run ends
+    const size_t o_items = off;
+    off = up256(off + (inl ? 0u : n_items * sizeof(tsr::FaItem) + 8u * (size_t)T + 4u * map_words));
+    const size_t o_xq = off; off = up256(off + (n_map ? (size_t)T * K : 0u));
+    const size_t o_xd = off; off = up256(off + (n_map ? (size_t)T * K / 8u : 0u));
     const size_t o_S = off; off = up256(off + 4u * (size_t)w.cells * n_head);
     const size_t o_Mp = off; off = up256(off + 4u * (size_t)w.n_tiles * n_head);
     const size_t o_OP = off; off = up256(off + 4u * n_items * kC * n_head * D);
@@ -469,9 +491,18 @@ static int fa_unplanned(tsr_hip_ctx * ctx, const float * q_dev, uint32_t T, uint
         std::copy(w.items.begin(), w.items.end(), p.items);
         for (uint32_t t = 0; t < T; ++t) { p.tok_first[t] = w.tok[t]; p.tok_count[t] = w.tok[T + t]; }
     } else if constexpr (!NOALLOC) {                              // items | tok_first | tok_count, one copy
-        packed.resize(n_items * sizeof(tsr::FaItem) + 8u * (size_t)T);
+        packed.resize(n_items * sizeof(tsr::FaItem) + 8u * (size_t)T + 4u * map_words);
         memcpy(packed.data(), w.items.data(), n_items * sizeof(tsr::FaItem));
         memcpy(packed.data() + n_items * sizeof(tsr::FaItem), w.tok.data(), 8u * (size_t)T);
+        if (n_map != 0u) {
+            uint32_t * m = (uint32_t *)(packed.data() + n_items * sizeof(tsr::FaItem) + 8u * (size_t)T);
+            std::fill(m, m + (size_t)n_map * T, 0xFFFFFFFFu);
+            for (size_t i = 0; i < n_items; ++i) {
+                const tsr::FaItem & it = w.items[i];
+                for (uint32_t k = 0, a0 = (it.u0 - lo / 16u) / 16u; k < it.ntiles; ++k) m[(size_t)(a0 + k) * T + it.t] = (uint32_t)i;
+            }
+            for (uint32_t t = 0; t < T; ++t) m[(size_t)n_map * T + t] = msum[8u + 4u * t + 1u];
+        }
     }
 
     std::lock_guard<std::mutex> lk(ctx->mtx);
@@ -505,6 +536,17 @@ static int fa_unplanned(tsr_hip_ctx * ctx, const float * q_dev, uint32_t T, uint
     a.OP = (float *)(base + o_OP);
     a.LP = (float *)(base + o_LP);
     a.max_groups = w.max_groups;
+    if (n_map != 0u) {
+        a.tmap = a.tok_count + T;
+        a.hi = a.tmap + (size_t)n_map * T;
+        a.n_map = n_map;
+        a.u_lo = lo / 16u;
+        a.lo = lo;
+        a.xq = base + o_xq;
+        a.xd = (const float *)(base + o_xd);
+        a.s_bytes = (uint32_t)(4u * w.cells * n_head);
+        if (tsr_launch_qact_mm(q_dev, q_stride, K, T, base + o_xq, (float *)(base + o_xd), s)) return TSR_HIP_E_HIP;
+    }
     ctx->ctr.flash_attn_calls++;
     ctx->ctr.flash_attn_kv_bytes += w.cells * (uint64_t)E / 32u * 34u * 2u;
     return tsr_launch_fa(a, p, T, (uint32_t)ctx->n_cu, s) ? TSR_HIP_E_HIP : TSR_HIP_OK;

@@ -83,6 +83,42 @@ def test_fa_causal_prefill_baseline_512(dev, oc):
     assert_bits_equal(got, want, "causal prefill 512")
 
 
+@pytest.mark.parametrize("T,lo,hist,n_head,n_head_kv,D,special", [
+    (40, 0, 2290, 64, 8, 128, None),      # 9 tiles and a part, a ragged second row block
+    (33, 37, 2600, 64, 8, 128, None),     # the runs start inside a group, chunk cuts from there
+    (70, 0, 2500, 64, 1, 64, None),       # D 64, one KV head
+    (9, 0, 9300, 64, 8, 128, None),       # one row block of 9 rows, several chunks a row
+    (40, 0, 2290, 64, 8, 128, "scales"),  # NaN / Inf / largest scales of K and V, zero and NaN queries
+], ids=["ragged", "lo37", "d64", "t9", "special"])
+def test_fa_rows_matrix_core_scores(dev, oc, T, lo, hist, n_head, n_head_kv, D, special):
+    """Many rows with one run each from a common cell: enough scores (n_head x cells x D / 64 >= 10 x 2^20)
+    for the matrix-core score kernel. Row t sees cells [lo, hist + t], the rows' cells planned newest last."""
+    n, E = hist + T, n_head_kv * D
+    assert sum((hist + t + 16) // 16 * 16 - lo // 16 * 16 for t in range(T)) * n_head * (D // 64) >= 10 << 20
+    kc, vc = _cache(oc, n, E, T + D)
+    q = S.normal(T, T * n_head * D).reshape(T, n_head * D)
+    if special:
+        k, v = kc.reshape(n, E // 32, 34), vc.reshape(n, E // 32, 34)
+        for row, b, bits in ((5, 1, 0x7C00), (300, 9, 0xFC00), (901, 17, 0x7E00), (1500, 26, 0x7BFF)):
+            k[row, b, :2] = np.array([bits], np.uint16).view(np.uint8)
+            v[row + 1, b, :2] = np.array([bits], np.uint16).view(np.uint8)
+        v[:, 30, :2] = np.array([0x0001], np.uint16).view(np.uint8)       # the smallest scale: tiny weights
+        q[3, :128], q[7, 640] = 0.0, np.nan
+        q[11] *= np.float32(60.0)                                         # most weights underflow to zero
+    msum = np.zeros(8 + 4 * T, np.uint32)
+    msum[0], msum[1], msum[2] = 0x4D55534D, T, n
+    msum[8::4], msum[9::4] = lo, hist + 1 + np.arange(T)
+    scale = np.float32(1.0 / math.sqrt(D))
+    want = oc.flash_attn(q, kc, vc, D, n_head, n_head_kv, scale, msum, None, [[hist, n]])
+    K_, V_ = dev.kv(E, n), dev.kv(E, n)
+    K_.set_bytes(0, kc)
+    V_.set_bytes(1, vc)
+    out = dev.alloc(4 * T * n_head * D)
+    dev.flash_attn(dev.upload(q), T, n_head * D, K_, V_, D, n_head, n_head_kv, scale, msum, out, n_head * D,
+                   new_runs=[[hist, n]])
+    assert_bits_equal(out.read(np.float32, (T, n_head * D)), want, f"{T} rows behind {hist}")
+
+
 def test_fa_general_and_two_run_masks(dev, oc):
     m2 = np.zeros((3, 100), np.float16); m2[:, 10:20] = -2.5; m2[1, 50:] = -np.inf
     got, want = _fa(dev, oc, 100, 112, 8, 2, 64, T=3, mask=m2)
