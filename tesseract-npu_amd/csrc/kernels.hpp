@@ -224,6 +224,8 @@ int tsr_launch_qact(const tsr::QactArgs & a, uint32_t T, hipStream_t s);
 uint32_t tsr_wl_rows_per_block(uint32_t fmt, uint32_t N, uint32_t K, uint32_t n_cu);
 int tsr_launch_mv_q8_0(const tsr::MvArgs & a, hipStream_t s);
 int tsr_launch_mv_q4_k(const tsr::MvArgs & a, hipStream_t s);
+// several token rows, up to 15 a workgroup (k_matrows.hip); every option of the matvec but isums
+int tsr_launch_mr(const tsr::MvArgs & a, bool q4k, hipStream_t s);
 int tsr_launch_qact_mm(const float * x, uint64_t x_stride, uint32_t K, uint32_t T, uint8_t * xq, float * xd,
                        hipStream_t s);
 int tsr_launch_mm_q8_0(const tsr::MmArgs & a, hipStream_t s);

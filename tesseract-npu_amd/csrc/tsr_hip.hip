@@ -475,7 +475,7 @@ static int mul_mat_locked(tsr_hip_ctx * ctx, const tsr_hip_weight * w, const flo
     if (w == nullptr || x_dev == nullptr || y_dev == nullptr || T == 0u) return TSR_HIP_E_ARG;
     const bool glu = (flags & TSR_HIP_MM_GLU) != 0u;
     if (prep != nullptr || glu) {
-        // the fused forms run on the matvec kernels (not the matrix-core prefill shapes); the norm needs
+        // the fused forms run on the matvec and few-row kernels (not Q8_0's prefill shapes); the norm needs
         // the whole row in one round of loads: K <= 8192; GLU pairs whole rows in every row block
         if ((prep != nullptr && w->K > 8192u) || (T >= kMmMinTokens && w->fmt == TSR_HIP_FMT_Q8_0) ||
             (glu && ((w->N & 1u) || (w->rb & 1u))))
@@ -548,7 +548,7 @@ static int mul_mat_locked(tsr_hip_ctx * ctx, const tsr_hip_weight * w, const flo
         return TSR_HIP_OK;
     }
     // prefill: T >= 16 tokens of Q4_K on the matrix cores (QACT A256 of every token into scratch,
-    // block-major), with the GLU epilogue when asked; the fused norm form stays on the matvec kernels
+    // block-major), with the GLU epilogue when asked; the fused norm form stays on the few-row kernels
     if (T >= kMmMinTokens && w->fmt == TSR_HIP_FMT_Q4_K && isums == nullptr && prep == nullptr) {
         const uint32_t chunk = std::min(T, kMmChunk), tpc = (chunk + 31u) & ~31u;
         const size_t s_off = ((size_t)chunk * w->K + 255u) & ~(size_t)255u;
@@ -582,13 +582,20 @@ static int mul_mat_locked(tsr_hip_ctx * ctx, const tsr_hip_weight * w, const flo
         }
         return TSR_HIP_OK;
     }
+    // The matvec (one row; the integer sums; a workgroup per row and row block) or, for several rows, k_matrows.hip
+    // (the weights once per 15 rows; the fused norm form comes here at any T). As long as the matvec's
+    // workgroups run side by side, one a CU, it is the faster one: Q4_K 1024x2048, 4 rows 4.3 us against 4.9;
+    // beyond that it never is: 2048x2048, 3 rows 7.1 against 4.8, Q8_0 4096x4096, 2 rows 8.2 against 7.5.
+    const uint32_t blocks = (w->N + w->rb - 1u) / w->rb;
+    const bool rows = isums == nullptr && (uint64_t)blocks * T > ctx->n_cu && T > 1u;
     for (uint32_t t0 = 0; t0 < T; t0 += 65535u) {
         const uint32_t tt = std::min(T - t0, 65535u);
         a.x = x_dev + (size_t)t0 * x_stride;
         a.y = y_dev + (size_t)t0 * y_stride;
         a.add = add_dev ? add_dev + (size_t)t0 * add_stride : nullptr;
         a.T = tt;
-        const int rc = w->fmt == TSR_HIP_FMT_Q8_0 ? tsr_launch_mv_q8_0(a, s) : tsr_launch_mv_q4_k(a, s);
+        const bool q4k = w->fmt == TSR_HIP_FMT_Q4_K;
+        const int rc = rows && tt > 1u ? tsr_launch_mr(a, q4k, s) : (q4k ? tsr_launch_mv_q4_k(a, s) : tsr_launch_mv_q8_0(a, s));
         if (rc) return rc == -2 ? TSR_HIP_E_SHAPE : TSR_HIP_E_HIP;
     }
     return TSR_HIP_OK;

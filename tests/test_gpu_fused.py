@@ -135,6 +135,53 @@ def test_mul_mat_glu(dev, oc, fmt, F, K, T, norm):
     wt.free()
 
 
+@pytest.mark.parametrize("fmt,N,K,T,opt", [
+    (H.FMT_Q4_K, 4100, 256, 2, "acc"),      # one super-block: 15 waves without terms
+    (H.FMT_Q4_K, 4127, 4352, 3, "add"),     # odd rows; a second super-block for one wave, loaded as a pair
+    (H.FMT_Q4_K, 8222, 4096, 9, "none"),    # a tile of fewer rows; the 16-token form
+    (H.FMT_Q4_K, 10000, 8448, 12, "none"),  # row chunks that quantize again, groups of super-blocks
+    (H.FMT_Q4_K, 4098, 16640, 5, "none"),   # groups of the 8-token form
+    (H.FMT_Q4_K, 20000, 2048, 15, "glu"),   # row chunks over one quantization
+    (H.FMT_Q4_K, 5000, 1024, 31, "norm"),   # shares of 11, 11 and 9 tokens
+    (H.FMT_Q4_K, 4130, 8192, 8, "norm"),
+    (H.FMT_Q8_0, 4100, 32, 2, "acc"),       # one block
+    (H.FMT_Q8_0, 4127, 1056, 4, "add"),     # odd rows; three blocks for one wave
+    (H.FMT_Q8_0, 8222, 544, 7, "none"),
+    (H.FMT_Q8_0, 20000, 1024, 9, "glu"),    # row chunks over one quantization
+    (H.FMT_Q8_0, 16900, 8224, 9, "none"),   # row chunks that quantize again, groups of blocks
+    (H.FMT_Q8_0, 4098, 16416, 3, "none"),   # groups of the 8-token form
+    (H.FMT_Q8_0, 4130, 8192, 15, "norm"),
+], ids=lambda v: str(v))
+def test_few_rows(dev, oc, fmt, N, K, T, opt):
+    """The kernels of several token rows over more row blocks than the card has CUs / T, at the edges of their
+    tiles, groups and chunks, with rows of special values, of scales below 2^-60 and of equal values."""
+    print(f"\nfew rows fmt {fmt} {N}x{K} T {T} {opt}", flush=True)
+    blocks = S.quant_rows(fmt, S.seed_of("few-rows", f"{fmt}-{N}-{K}"), N, K)
+    x = _x_rows(K, T, N + K + T)
+    x[-1] *= np.float32(1e-22)
+    if T > 3:
+        x[2] = 0.0
+        x[3] = 0.75
+    rng = np.random.default_rng(N)
+    nw = (1.0 + 0.1 * rng.standard_normal(K)).astype(np.float32)
+    c = rng.standard_normal((T, N)).astype(np.float32)
+    xn = oc.rms_norm(x, 1e-5, nw[None]) if opt == "norm" else x
+    want = oc.mul_mat(fmt, blocks, K, xn, add=c if opt in ("add", "acc") else None, threads=8)
+    if opt == "glu":
+        want = oc.swiglu(np.ascontiguousarray(want[:, 0::2]), np.ascontiguousarray(want[:, 1::2]))
+    wt = dev.weight(fmt, blocks, N, K)
+    n = want.shape[1]
+    xb, yb = dev.upload(x), dev.upload(c)
+    if opt == "norm":
+        dev.mul_mat_norm(wt, xb, T, K, 1e-5, dev.upload(nw), yb, n)
+    elif opt == "add":
+        dev.mul_mat(wt, xb, T, K, yb, n, add=dev.upload(c), add_stride=N)
+    else:
+        dev.mul_mat(wt, xb, T, K, yb, n, flags={"acc": H.MM_ACC_DST, "glu": H.MM_GLU}.get(opt, 0))
+    assert_bits_equal(yb.read(np.float32, (T, n)), want, opt)
+    wt.free()
+
+
 def test_fused_shape_refusals(dev):
     blocks = S.quant_rows(H.FMT_Q4_K, 1, 16, 16384)
     wt = dev.weight(H.FMT_Q4_K, blocks, 16, 16384)
