@@ -40,6 +40,13 @@ __global__ void k_kv_bytes(KvArgs a, uint32_t which, uint64_t off, uint64_t n, u
     else stage[i] = a.base[d];
 }
 
+// A work list from pinned host memory, read over the bus by a kernel in stream order. An engine copy of 20 KB in
+// front of FLASH_ATTN_EXT left the compute queue idle for 18 us (two hand-overs between the engines).
+__global__ __launch_bounds__(256) void k_fetch(uint4 * dst, const uint4 * host, uint32_t n16) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i < n16) dst[i] = host[i];
+}
+
 // SET_ROWS: one wave per 256 values of a row (8 A32 blocks), grid (ceil(E/256), n_rows).
 __global__ __launch_bounds__(64) void k_kv_set_rows(KvArgs a, uint32_t which, const float * src, uint64_t src_stride,
                                                     const int64_t * idx, int32_t * bad) {
@@ -65,6 +72,13 @@ int tsr_launch_kv_bytes(const tsr::KvArgs & a, uint32_t which, uint64_t off, uin
     if (n == 0) return 0;
     const uint64_t blocks = (n + 255u) / 256u;
     hipLaunchKernelGGL(tsr::k_kv_bytes, dim3((uint32_t)blocks), dim3(256), 0, s, a, which, off, n, stage, to_dev);
+    return hipGetLastError() == hipSuccess ? 0 : -4;
+}
+
+int tsr_launch_fetch(void * dst, const void * host, size_t bytes, hipStream_t s) {
+    const uint32_t n16 = (uint32_t)((bytes + 15u) / 16u);
+    if (n16 == 0u) return 0;
+    hipLaunchKernelGGL(tsr::k_fetch, dim3((n16 + 255u) / 256u), dim3(256), 0, s, (uint4 *)dst, (const uint4 *)host, n16);
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 

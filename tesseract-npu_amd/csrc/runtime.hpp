@@ -121,6 +121,53 @@ struct tsr_staging {
     }
 };
 
+// Pinned host slots for the work lists of unplanned FLASH_ATTN_EXT calls: the list is built in a slot and a
+// kernel reads it from there into the scratch (tsr_launch_fetch). A slot is reused only after the kernel that
+// last read it has run (its event). Allocated at the first list (1 MB a context), given back with the context;
+// a list beyond a slot, or a context without the memory, takes a copy of pageable memory instead.
+struct tsr_lists {
+    static constexpr uint32_t kSlots = 4;
+    static constexpr size_t kSlotBytes = (size_t)256 << 10;
+    uint8_t * host = nullptr;
+    hipEvent_t ev[kSlots] = {};
+    bool used[kSlots] = {};
+    bool tried = false;
+    uint32_t next = 0;
+    uint8_t * acquire(size_t bytes) {                             // nullptr: none for this list
+        if (bytes > kSlotBytes) return nullptr;
+        if (!tried) {
+            tried = true;
+            bool ok = hipHostMalloc((void **)&host, kSlots * kSlotBytes, hipHostMallocCoherent) == hipSuccess;
+            for (uint32_t i = 0; ok && i < kSlots; ++i) ok = hipEventCreateWithFlags(&ev[i], hipEventDisableTiming) == hipSuccess;
+            if (!ok) {
+                (void)hipGetLastError();
+                release();
+            }
+        }
+        if (host == nullptr) return nullptr;
+        if (used[next] && hipEventSynchronize(ev[next]) != hipSuccess) return nullptr;
+        return host + next * kSlotBytes;
+    }
+    int send(void * dst_dev, size_t bytes, hipStream_t s) {       // the slot acquired last
+        const uint32_t k = next;
+        next = (next + 1u) % kSlots;
+        if (tsr_launch_fetch(dst_dev, host + k * kSlotBytes, bytes, s)) return TSR_HIP_E_HIP;
+        const int rc = tsr::hip_err(hipEventRecord(ev[k], s), "hipEventRecord list");
+        used[k] = rc == 0;
+        return rc;
+    }
+    void release() {
+        for (uint32_t i = 0; i < kSlots; ++i) {
+            if (ev[i] && used[i]) (void)hipEventSynchronize(ev[i]);
+            if (ev[i]) (void)hipEventDestroy(ev[i]);
+            ev[i] = nullptr;
+            used[i] = false;
+        }
+        if (host) (void)hipHostFree(host);
+        host = nullptr;
+    }
+};
+
 struct tsr_hip_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -131,6 +178,7 @@ struct tsr_hip_ctx {
     tsr_hip_counters ctr{};
     tsr_scratch scratch;
     tsr_staging staging;
+    tsr_lists lists;
     tsr::ExpkTab expk{};
     uint32_t fa_spin_max = 1u << 20;    // polls of the fused decode FA's tile-key wait (s_sleep 1 each)
     uint8_t * fa_fixed = nullptr;       // device address of this device's fixed FA array (tsr_fa_fixed_init)

@@ -486,24 +486,24 @@ static int fa_unplanned(tsr_hip_ctx * ctx, const float * q_dev, uint32_t T, uint
     tsr::FaPlan p{};
     p.n_items = (uint32_t)n_items;
     p.maxtiles = w.maxtiles;
-    std::vector<uint8_t> packed;
     if (inl) {
         std::copy(w.items.begin(), w.items.end(), p.items);
         for (uint32_t t = 0; t < T; ++t) { p.tok_first[t] = w.tok[t]; p.tok_count[t] = w.tok[T + t]; }
-    } else if constexpr (!NOALLOC) {                              // items | tok_first | tok_count, one copy
-        packed.resize(n_items * sizeof(tsr::FaItem) + 8u * (size_t)T + 4u * map_words);
-        memcpy(packed.data(), w.items.data(), n_items * sizeof(tsr::FaItem));
-        memcpy(packed.data() + n_items * sizeof(tsr::FaItem), w.tok.data(), 8u * (size_t)T);
-        if (n_map != 0u) {
-            uint32_t * m = (uint32_t *)(packed.data() + n_items * sizeof(tsr::FaItem) + 8u * (size_t)T);
-            std::fill(m, m + (size_t)n_map * T, 0xFFFFFFFFu);
-            for (size_t i = 0; i < n_items; ++i) {
-                const tsr::FaItem & it = w.items[i];
-                for (uint32_t k = 0, a0 = (it.u0 - lo / 16u) / 16u; k < it.ntiles; ++k) m[(size_t)(a0 + k) * T + it.t] = (uint32_t)i;
-            }
-            for (uint32_t t = 0; t < T; ++t) m[(size_t)n_map * T + t] = msum[8u + 4u * t + 1u];
-        }
     }
+    // items | tok_first | tok_count (| tile map | run ends)
+    const size_t list_bytes = n_items * sizeof(tsr::FaItem) + 8u * (size_t)T + 4u * map_words;
+    auto pack = [&](uint8_t * list) {
+        memcpy(list, w.items.data(), n_items * sizeof(tsr::FaItem));
+        memcpy(list + n_items * sizeof(tsr::FaItem), w.tok.data(), 8u * (size_t)T);
+        if (n_map == 0u) return;
+        uint32_t * m = (uint32_t *)(list + n_items * sizeof(tsr::FaItem) + 8u * (size_t)T);
+        std::fill(m, m + (size_t)n_map * T, 0xFFFFFFFFu);
+        for (size_t i = 0; i < n_items; ++i) {
+            const tsr::FaItem & it = w.items[i];
+            for (uint32_t k = 0, a0 = (it.u0 - lo / 16u) / 16u; k < it.ntiles; ++k) m[(size_t)(a0 + k) * T + it.t] = (uint32_t)i;
+        }
+        for (uint32_t t = 0; t < T; ++t) m[(size_t)n_map * T + t] = msum[8u + 4u * t + 1u];
+    };
 
     std::lock_guard<std::mutex> lk(ctx->mtx);
     (void)hipSetDevice(ctx->device);
@@ -520,7 +520,14 @@ static int fa_unplanned(tsr_hip_ctx * ctx, const float * q_dev, uint32_t T, uint
             // a host-to-device copy of a host vector cannot be recorded into a graph (the vector is gone
             // when the graph replays): long work lists are for eager calls or a tsr_hip_fa_plan
             if (tsr_capturing(s)) return TSR_HIP_E_ARG;
-            rc = hip_err(hipMemcpyAsync(base + o_items, packed.data(), packed.size(), hipMemcpyHostToDevice, s), "fa plan");
+            if (uint8_t * slot = ctx->lists.acquire(list_bytes)) {
+                pack(slot);
+                rc = ctx->lists.send(base + o_items, list_bytes, s);
+            } else {
+                std::vector<uint8_t> packed(list_bytes);
+                pack(packed.data());
+                rc = hip_err(hipMemcpyAsync(base + o_items, packed.data(), list_bytes, hipMemcpyHostToDevice, s), "fa plan");
+            }
             if (rc) return rc;
         }
     }

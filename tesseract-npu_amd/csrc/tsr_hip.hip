@@ -132,6 +132,7 @@ int tsr_hip_close(tsr_hip_ctx * ctx) {
         (void)hipStreamSynchronize(ctx->stream);
         ctx->scratch.release();
         ctx->staging.release();
+        ctx->lists.release();
         if (ctx->flags_dev) (void)hipFree(ctx->flags_dev);
         (void)hipStreamDestroy(ctx->stream);
     }

@@ -206,6 +206,18 @@ class Buffer:
             pass
 
 
+class BufferPart(Buffer):
+    """nbytes of a Buffer from offset on: addressed like a buffer of its own, freed with the whole one."""
+
+    def __init__(self, whole: Buffer, offset: int, nbytes: int):
+        if offset + nbytes > whole.nbytes:
+            raise ValueError("a part beyond the buffer")
+        self.dev, self.nbytes, self.whole, self.ptr = whole.dev, int(nbytes), whole, whole.ptr + offset
+
+    def free(self) -> None:
+        self.ptr = self.whole = None
+
+
 class Weight:
     def __init__(self, dev: "Device", fmt: int, blocks, N: int, K: int):
         self.dev, self.fmt, self.N, self.K = dev, fmt, N, K

@@ -185,11 +185,14 @@ class LlamaDecoder:
         self.att = dev.alloc(c.n_q * f4)
         self.gu = dev.alloc(2 * c.n_ff * f4)
         self.glu = dev.alloc(c.n_ff * f4)
-        self.logits = dev.alloc(c.n_vocab * f4)
-        self.tok = dev.alloc(4)            # int32 token id of the step (GET_ROWS ids)
+        # what the host reads after a step lies together (one copy each way: a copy and its wait take ~20 us)
+        self._out = dev.alloc(c.n_vocab * f4 + 4)
+        self.logits = H.BufferPart(self._out, 0, c.n_vocab * f4)
+        self.bad = H.BufferPart(self._out, c.n_vocab * f4, 4).fill(0)
         self.next = dev.alloc(4)           # int32 greedy token (ARGMAX) of an eager step
-        self.params = dev.alloc(16)        # int32 position (ROPE) at 0, int64 cell (SET_ROWS_KV) at 8
-        self.bad = dev.alloc(4).fill(0)
+        # int32 position (ROPE) at 0, int64 cell (SET_ROWS_KV) at 8, int32 token id (GET_ROWS ids) at 16
+        self.params = dev.alloc(24)
+        self.tok = H.BufferPart(self.params, 16, 4)
         self.rtab = dev.alloc(4 * c.head_dim)  # ROPE angles of the token's position (tsr_hip_rope_table)
         self.scale = 1.0 / math.sqrt(c.head_dim)
         self.plan = dev.fa_plan(c.head_dim, c.n_head, c.n_head_kv, 1, kv_size)
@@ -230,8 +233,10 @@ class LlamaDecoder:
         self._pf = {"U": U, "x": d.alloc(U * c.n_embd * f4), "h": d.alloc(U * c.n_embd * f4),
                     "xn": d.alloc(U * c.n_embd * f4), "qkv": d.alloc(U * (c.n_q + 2 * c.E) * f4),
                     "att": d.alloc(U * c.n_q * f4), "gu": d.alloc(U * 2 * c.n_ff * f4),
-                    "glu": d.alloc(U * c.n_ff * f4), "ids": d.alloc(U * 4), "pos": d.alloc(U * 4),
-                    "cell": d.alloc(U * 8)}
+                    "glu": d.alloc(U * c.n_ff * f4), "in": d.alloc(U * 16)}
+        # a ubatch's cells (int64), positions and token ids (int32), written with one copy
+        self._pf.update(cell=H.BufferPart(self._pf["in"], 0, U * 8), pos=H.BufferPart(self._pf["in"], U * 8, U * 4),
+                        ids=H.BufferPart(self._pf["in"], U * 12, U * 4))
         return self._pf
 
     def prefill(self, tokens, pos0: int = 0, ubatch: int = 512) -> None:
@@ -266,10 +271,15 @@ class LlamaDecoder:
         w3, f4 = nq + 2 * E, 4
         pf = self._prefill_buffers(T)
         x, h, xn, qkv, att, gu, glu = (pf[k] for k in ("x", "h", "xn", "qkv", "att", "gu", "glu"))
-        pos = pos0 + np.arange(T, dtype=np.int64)
-        pf["ids"].write(toks)
-        pf["pos"].write(pos.astype(np.int32))
-        pf["cell"].write(pos)
+        U, pos = pf["U"], pos0 + np.arange(T, dtype=np.int64)
+        ins = np.zeros(4 * U, np.int32)
+        ins[:2 * T].view(np.int64)[:] = pos
+        ins[2 * U:2 * U + T] = pos
+        ins[3 * U:3 * U + T] = toks
+        if ins.nbytes <= 16384:                                   # queued behind the ubatch before, no wait
+            d.write_async(pf["in"], ins)
+        else:
+            pf["in"].write(ins)
         n_kv = min(self.kv_size, (pos0 + T + 255) // 256 * 256)
         msum, runs = msum_causal(pos0, T, n_kv), np.array([[pos0, pos0 + T]], np.uint32)
         # 16 or more tokens run the MUL_MATs on the matrix cores, which take no fused RMS_NORM: there the
@@ -323,11 +333,12 @@ class LlamaDecoder:
         return msum_decode(pos, n_kv), np.array([[pos, pos + 1]], np.uint32)
 
     @staticmethod
-    def _params(pos: int) -> np.ndarray:
-        p = np.zeros(2, np.int64)
-        p[1] = pos
-        v = p.view(np.int32)
-        v[0] = pos
+    def _params(pos: int, token: int | None = None) -> np.ndarray:
+        """The bytes of self.params, up to the token when one is given."""
+        p = np.zeros(4 if token is None else 5, np.int32)
+        p[0] = p[2] = pos                  # positions are below 2^31: the high word of the cell is 0
+        if token is not None:
+            p[4] = token
         return p
 
     def _ops(self, out_tok, msum=None, runs=None, stream=None) -> None:
@@ -402,14 +413,12 @@ class LlamaDecoder:
 
     def step_graph(self, token: int | None, pos: int, n_kv: int | None = None) -> None:
         """One decode token as one graph replay. Per token the host only plans the attention chunks and
-        queues two small stream-ordered copies (position / cell and the plan); the greedy token of the
+        queues two small stream-ordered copies (position / cell / token and the plan); the greedy token of the
         previous replay is embedded from the device (token None). The graph is captured on the first
         call and again whenever the plan's shape changes. Nothing waits for the device."""
         d = self.dev
         msum, runs = self._mask(pos, n_kv)
-        if token is not None:
-            d.write_async(self.tok, np.array([token], np.int32))
-        d.write_async(self.params, self._params(pos))
+        d.write_async(self.params, self._params(pos, token))
         changed = self.plan.set(msum, runs)
         if self.graph is None or changed:
             if self.graph is not None:
@@ -429,9 +438,7 @@ class LlamaDecoder:
         Nothing waits for the device."""
         d = self.dev
         msum, runs = self._mask(pos, n_kv)
-        if token is not None:
-            d.write_async(self.tok, np.array([token], np.int32))
-        d.write_async(self.params, self._params(pos))
+        d.write_async(self.params, self._params(pos, token))
         self.plan.set(msum, runs)
         self._ops(self.tok)
 
@@ -454,8 +461,9 @@ class LlamaDecoder:
         nothing); bit 1, a bounded wait of the one-launch FLASH_ATTN_EXT expired; bit 2, one of its
         workgroups ran on another XCD than its KV head's (for bits 1 and 2 the attention output is not
         valid). The flag is cleared when it is reported."""
-        self.dev.sync()
-        bad = int(self.bad.read(np.int32, (1,))[0])
+        self._check_flag(int(self.bad.read(np.int32, (1,))[0]))   # read waits for the stream's work
+
+    def _check_flag(self, bad: int) -> None:
         if bad == 0:
             return
         self.bad.fill(0)
@@ -471,8 +479,9 @@ class LlamaDecoder:
 
     def read_logits(self) -> np.ndarray:
         """The logits of the last step (checked: raises DecodeError on a raised flag)."""
-        self.check()
-        return self.logits.read(np.float32, (self.cfg.n_vocab,))
+        out = self._out.read(np.float32, (self.cfg.n_vocab + 1,))
+        self._check_flag(int(out[-1:].view(np.int32)[0]))
+        return out[:-1]
 
     def read_next(self) -> int:
         """The greedy token of the last eager step (checked)."""

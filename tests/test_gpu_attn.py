@@ -119,6 +119,29 @@ def test_fa_rows_matrix_core_scores(dev, oc, T, lo, hist, n_head, n_head_kv, D, 
     assert_bits_equal(out.read(np.float32, (T, n_head * D)), want, f"{T} rows behind {hist}")
 
 
+@pytest.mark.parametrize("T,calls", [(40, 11), (7000, 2)], ids=["slots_reused", "list_beyond_a_slot"])
+def test_fa_queued_work_lists(dev, oc, T, calls):
+    """Unplanned calls with work lists of their own queued behind each other without a wait: each sees its own
+    list, also when the pinned slots wrap (4) and when a list does not fit one (256 KB)."""
+    n, nh, nkv, D = 300, 2, 1, 64
+    kc, vc = _cache(oc, n, nkv * D, T)
+    K_, V_ = dev.kv(nkv * D, n), dev.kv(nkv * D, n)
+    K_.set_bytes(0, kc)
+    V_.set_bytes(1, vc)
+    q = S.normal(T + 1, T * nh * D).reshape(T, nh * D)
+    qb, outs, masks = dev.upload(q), [dev.alloc(4 * T * nh * D) for _ in range(calls)], []
+    for i in range(calls):
+        m = np.zeros(8 + 4 * T, np.uint32)
+        m[0], m[1], m[2] = 0x4D55534D, T, n
+        m[8::4] = np.arange(T) % 7 + i
+        m[9::4] = m[8::4] + 1 + (np.arange(T) * (i + 3)) % 120
+        masks.append(m)
+        dev.flash_attn(qb, T, nh * D, K_, V_, D, nh, nkv, 0.125, m, outs[i], nh * D)
+    for i, m in enumerate(masks):
+        want = oc.flash_attn(q, kc, vc, D, nh, nkv, np.float32(0.125), m, None, [])
+        assert_bits_equal(outs[i].read(np.float32, (T, nh * D)), want, f"call {i}")
+
+
 def test_fa_general_and_two_run_masks(dev, oc):
     m2 = np.zeros((3, 100), np.float16); m2[:, 10:20] = -2.5; m2[1, 50:] = -np.inf
     got, want = _fa(dev, oc, 100, 112, 8, 2, 64, T=3, mask=m2)
