@@ -97,6 +97,63 @@ __global__ __launch_bounds__(128) void k_rms_norm(const float * x, uint64_t x_st
     }
 }
 
+// The same for rows of at most 4096 values in whole, aligned float4s (the launcher's rule): 256 threads hold the
+// row and its weights, a quarter of the loads a thread; the squares pass through LDS to the 128 chains of waves 0
+// and 1, and every wave forms the scale itself from the two halves. Bound by its latencies (load, 32 additions in
+// order, tree, divisions): 300 rows of 4096 8.6 -> 6.0 us, 256 rows of 2048 6.4 -> 4.1.
+__global__ __launch_bounds__(256) void k_rms_norm4(const float * x, uint64_t x_stride, uint32_t n, float eps, float inv_n,
+                                                   const float * w, uint64_t w_stride, uint32_t w_period, float * y,
+                                                   uint64_t y_stride) {
+    __shared__ __align__(16) float s_q[4096];
+    __shared__ float s_half[2];
+    const uint32_t r = blockIdx.x, i = threadIdx.x;
+    const float * xr = x + (size_t)r * x_stride;
+    const bool has_w = w != nullptr;
+    const float * wr = has_w ? w + (size_t)(r % w_period) * w_stride : xr;
+    float4 v[4], wv[4];
+#pragma unroll
+    for (uint32_t c = 0; c < 4u; ++c) {
+        const uint32_t j = 4u * i + 1024u * c;
+        v[c] = j < n ? *(const float4 *)(xr + j) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+#pragma unroll
+    for (uint32_t c = 0; c < 4u; ++c) {
+        const uint32_t j = 4u * i + 1024u * c;
+        wv[c] = j < n ? *(const float4 *)(wr + j) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+#pragma unroll
+    for (uint32_t c = 0; c < 4u; ++c) {
+        const uint32_t j = 4u * i + 1024u * c;
+        if (j < n) *(float4 *)(s_q + j) = sq4(v[c]);
+    }
+    __syncthreads();
+    if (i < 128u) {
+        float p = 0.0f;
+        for (uint32_t j0 = i; j0 < n; j0 += 1024u) {
+            float q[8];
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; ++k) q[k] = s_q[min(j0 + 128u * k, n - 1u)];
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; ++k)
+                if (j0 + 128u * k < n) p = p + q[k];              // = FA(p, FM(v, v)): see rms_tree64
+        }
+        p = rms_tree64(p);
+        if ((i & 63u) == 0u) s_half[i >> 6] = p;
+    }
+    __syncthreads();
+    const float s = rms_scale(s_half[0], s_half[1], inv_n, eps);
+    if (!prep_norm_apply_fast(v, s, wv, has_w)) {
+#pragma unroll
+        for (uint32_t c = 0; c < 4u; ++c) v[c] = prep_norm_apply(v[c], s, wv[c], has_w);
+    }
+    float * yr = y + (size_t)r * y_stride;
+#pragma unroll
+    for (uint32_t c = 0; c < 4u; ++c) {
+        const uint32_t j = 4u * i + 1024u * c;
+        if (j < n) *(float4 *)(yr + j) = v[c];
+    }
+}
+
 // ---- ROPE (sw/sim/tsr_ref_vu.c:308-376) -----------------------------------------------------------
 // Workgroup (token, group of kRopeHeads heads). Every thread first loads the pairs it rotates; one
 // lane runs the angle recurrence (rope_angles); the lanes then take sin / cos of the angles,
@@ -406,8 +463,12 @@ __global__ __launch_bounds__(64) void k_argmax_pick(const uint64_t * part, uint3
 // ---- launchers ------------------------------------------------------------------------------------
 int tsr_launch_rms_norm(const float * x, uint64_t x_stride, uint32_t n, uint32_t rows, float eps, float inv_n,
                         const float * w, uint64_t w_stride, uint32_t w_period, float * y, uint64_t y_stride, hipStream_t s) {
-    hipLaunchKernelGGL(tsr::k_rms_norm, dim3(rows), dim3(128), 0, s, x, x_stride, n, eps, inv_n, w, w_stride,
-                       w_period ? w_period : 1u, y, y_stride);
+    const uint32_t wp = w_period ? w_period : 1u;
+    auto whole = [](const void * p, uint64_t stride) { return ((uintptr_t)p & 15u) == 0u && (stride & 3u) == 0u; };
+    if (n <= 4096u && (n & 3u) == 0u && whole(x, x_stride) && whole(y, y_stride) && whole(w, w ? w_stride : 0u))
+        hipLaunchKernelGGL(tsr::k_rms_norm4, dim3(rows), dim3(256), 0, s, x, x_stride, n, eps, inv_n, w, w_stride, wp, y, y_stride);
+    else
+        hipLaunchKernelGGL(tsr::k_rms_norm, dim3(rows), dim3(128), 0, s, x, x_stride, n, eps, inv_n, w, w_stride, wp, y, y_stride);
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 

@@ -67,6 +67,22 @@ def test_rms_norm_strided_rows(dev, oc):
     assert (got[:, n:] == 7.0).all()
 
 
+@pytest.mark.parametrize("n", [4, 132, 1028, 2052, 4092])
+@pytest.mark.parametrize("off", [0, 1])
+def test_rms_norm_row_edges(dev, oc, n, off):
+    """Rows in whole float4s at the edges of the 256 threads, and (off 1) the same rows 4 bytes further on."""
+    rng = np.random.default_rng(n + off)
+    x = rng.standard_normal((3, n)).astype(np.float32)
+    x[1, :min(n, SPECIALS.size)] = SPECIALS[:n]
+    w = rng.standard_normal((2, n)).astype(np.float32)
+    flat = np.zeros(3 * n + 4, np.float32)
+    flat[off:off + 3 * n] = x.reshape(-1)
+    xb, yb = dev.upload(flat), dev.alloc(x.nbytes)
+    for wt in (w, None):
+        dev.rms_norm(xb.ptr + 4 * off, n, 3, n, 1e-5, yb, n, w=None if wt is None else dev.upload(w), w_stride=n, w_period=2)
+        assert_bits_equal(yb.read(np.float32, (3, n)), oc.rms_norm(x, 1e-5, wt, w_period=2 if wt is not None else 1), f"rms n={n}")
+
+
 @pytest.mark.parametrize("mode", [0, 2, 40])
 @pytest.mark.parametrize("hd,n_dims,nh", [(128, 128, 32), (128, 64, 8), (64, 64, 3), (256, 192, 4)])
 def test_rope(dev, oc, mode, hd, n_dims, nh):
