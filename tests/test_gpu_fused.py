@@ -723,3 +723,25 @@ def test_flash_attn_plan_rope_wait_expires(dev, oc):
     plan.free()
     kc.free()
     vc.free()
+
+
+@pytest.mark.parametrize("mode,n_dims", [(H.ROPE_NORMAL, 62), (H.ROPE_NORMAL, 32), (H.ROPE_NEOX, 24), (H.ROPE_NEOX, 20)],
+                         ids=lambda v: str(v))
+def test_rope_kv_partial_dims(dev, oc, mode, n_dims):
+    """Heads rotated in their first n_dims values only, in and out of whole units of four."""
+    T, hd, nh, nkv = 5, 64, 3, 1
+    E, nq = nkv * hd, nh * hd
+    x = np.random.default_rng(n_dims).standard_normal((T, nq + 2 * E)).astype(np.float32)
+    pos, cells = np.array([0, 3, 77, 511, 9000], np.int32), np.arange(5, dtype=np.int64) + 3
+    kc, vc = dev.kv(E, 32), dev.kv(E, 32)
+    kw, vw = np.zeros((32, E // 32 * 34), np.uint8), np.zeros((32, E // 32 * 34), np.uint8)
+    kc.set_bytes(0, kw)
+    vc.set_bytes(1, vw)
+    xb = dev.upload(x)
+    dev.rope_kv(xb, T, nq + 2 * E, hd, nh, nkv, n_dims, mode, dev.upload(pos), 10000.0, kc, vc, dev.upload(cells), None)
+    qk = oc.rope(np.ascontiguousarray(x[:, :nq + E]), pos, hd, n_dims, mode == H.ROPE_NEOX, theta_scale(10000.0, n_dims), 1.0,
+                 1.0, None)
+    assert_bits_equal(xb.read(np.float32, x.shape)[:, :nq + E], qk, "rotated q and k")
+    oc.kv_set_rows(kw, np.ascontiguousarray(qk[:, nq:]), cells)
+    oc.kv_set_rows(vw, np.ascontiguousarray(x[:, nq + E:]), cells)
+    assert (kc.get_bytes(0).reshape(32, -1) == kw).all() and (vc.get_bytes(1).reshape(32, -1) == vw).all()
