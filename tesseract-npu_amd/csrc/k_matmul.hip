@@ -251,14 +251,13 @@ __device__ __forceinline__ uint32_t q4k_sc(const uint4 mt, uint32_t j) {
     // meta bytes 4 + j: sc_j | (m_j & 3) << 6; nibble j of bytes 12..15: m_j >> 2 (wlayout.hpp)
     return __builtin_amdgcn_ubfe(j < 4u ? mt.y : mt.z, 8u * (j & 3u), 6);
 }
-// Work split. A workgroup of 4 waves computes a tile of 32 weight rows x 32 tokens. Wave j runs over the
-// super-blocks of PG = 4 consecutive partials, which are consecutive slots of the weight layout, and folds
-// each finished partial into its subtree of the 16-partial tree, parking the left halves of the two open
-// levels in LDS; the four subtrees meet in LDS at the end. (An empty partial is +0, and a sum that starts
+// Work split. A workgroup of W = 4 waves (8: see the launcher) computes a tile of 32 weight rows x 32 tokens.
+// Wave j runs over the super-blocks of PG = 16 / W consecutive partials, which are consecutive slots of the weight layout, and folds
+// each finished partial into its subtree of the 16-partial tree, parking the left halves of the open
+// levels in LDS; the W subtrees meet in LDS at the end. (An empty partial is +0, and a sum that starts
 // at +0 is never -0, so folding one in changes nothing. With at most 8 or 4 super-blocks the higher
-// partials are empty, and PG shrinks so that every wave has work.) Eight waves with two partials each and
-// all 16 partials in LDS, as this kernel had it, left a wave two super-blocks to set up and finish for and
-// every load to wait for.
+// partials are empty, and PG shrinks so that every wave has work.) Eight waves with every load waited for
+// and all 16 partials in LDS, as this kernel had it, left a wave two super-blocks to set up and finish for.
 //
 // Loads. A register is requested again for the next super-block right behind its last use, so that a load
 // has a super-block's work (~3 waves on the SIMD) to arrive. Every load is made on every path and in one
@@ -274,12 +273,11 @@ __device__ __forceinline__ uint32_t q4k_sc(const uint4 mt, uint32_t j) {
 //
 // GLU: weight rows 2j and 2j + 1 are the gate and up rows of output j, in adjacent lanes: the even lane
 // forms y = SWIGLU(gate, up) of the even tokens, the odd lane of the odd ones.
-constexpr uint32_t kMm4Waves = 4;
-template <bool GLU>
-__global__ __launch_bounds__(64 * kMm4Waves, 3) void k_mm_q4k(MmArgs a) {
-    constexpr int kLev = 2;                                        // open tree levels of a wave
-    __shared__ float4 s_p[kMm4Waves][kLev][4][64];                 // wave, level: values r = 4 q + e of a lane
-    __shared__ int s_slow[kMm4Waves];
+template <bool GLU, uint32_t W>
+__global__ __launch_bounds__(64 * W, W == 4u ? 3 : 2) void k_mm_q4k(MmArgs a) {
+    constexpr int kLev = W == 4u ? 2 : 1;                          // open tree levels of a wave
+    __shared__ float4 s_p[W][kLev][4][64];                         // wave, level: values r = 4 q + e of a lane
+    __shared__ int s_slow[W];
     const WGeom g = wgeom(a.N, a.K >> 8, a.rb, true);
     const uint32_t lane = __lane_id(), j = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     uint32_t tx, ty;
@@ -297,7 +295,7 @@ __global__ __launch_bounds__(64 * kMm4Waves, 3) void k_mm_q4k(MmArgs a) {
     const __amdgpu_buffer_rsrc_t rw = brsrc(a.w + wbase, (uint32_t)(wend - wbase));
     const __amdgpu_buffer_rsrc_t rx = brsrc(a.qa, a.d_off + 4u * a.tp * g.nb);
     const uint32_t np = g.nb > 8u ? 16u : (g.nb > 4u ? 8u : (g.nb > 2u ? 4u : g.nb));   // partials in use, a power of two
-    const uint32_t PG = max(np / kMm4Waves, 1u), w0 = PG * j;
+    const uint32_t PG = max(np / W, 1u), w0 = PG * j;
     const uint32_t sl0 = wl_slot(g, min(w0, 15u), 0u);
     const uint32_t sR = 16u * R, sG = 32u * R * g.nb;
     uint32_t owq = (uint32_t)(wl_quant_off(g, B, R, h, sl0, rr) - wbase);   // piece 2 gg + h: + sG gg; + sR per slot
@@ -445,28 +443,41 @@ __global__ __launch_bounds__(64 * kMm4Waves, 3) void k_mm_q4k(MmArgs a) {
     if constexpr (GLU) t64 = a.ex.t64[lane];
     lds_barrier();
 
-    // wave j finishes the value quad q = j: weight row n0 + lane % 32, tokens t0 + 8 j + 4 (lane / 32) + e
-    const bool any_slow = (s_slow[0] | s_slow[1] | s_slow[2] | s_slow[3]) != 0;
-    const float4 u0 = s_p[0][0][j][lane], u1 = s_p[1][0][j][lane], u2 = s_p[2][0][j][lane], u3 = s_p[3][0][j][lane];
-    auto tree4 = [&](float w0, float w1, float w2, float w3) {
-        return canon(any_slow ? sadd(sadd(w0, w1), sadd(w2, w3)) : (w0 + w1) + (w2 + w3));
-    };
-    const float v[4] = { tree4(u0.x, u1.x, u2.x, u3.x), tree4(u0.y, u1.y, u2.y, u3.y), tree4(u0.z, u1.z, u2.z, u3.z),
-                         tree4(u0.w, u1.w, u2.w, u3.w) };
-    const uint32_t nn = n0 + c, t4 = t0 + 8u * j + 4u * h;
+    // wave j finishes V values of each lane, r = V j + e: weight row n0 + lane % 32, tokens t4 + e
+    constexpr uint32_t V = 16u / W;
+    int any_slow = 0;
+    float u[W][V];
+#pragma unroll
+    for (uint32_t i = 0; i < W; ++i) {
+        any_slow |= s_slow[i];
+        const float * sp = (const float *)&s_p[i][0][V * j >> 2][lane] + (V * j & 3u);
+#pragma unroll
+        for (uint32_t e = 0; e < V; ++e) u[i][e] = sp[e];
+    }
+#pragma unroll
+    for (uint32_t m = W / 2u; m > 0u; m >>= 1)
+#pragma unroll
+        for (uint32_t i = 0; i < m; ++i)
+#pragma unroll
+            for (uint32_t e = 0; e < V; ++e)
+                u[i][e] = any_slow ? sadd(u[2u * i][e], u[2u * i + 1u][e]) : u[2u * i][e] + u[2u * i + 1u][e];
+    float v[V];
+#pragma unroll
+    for (uint32_t e = 0; e < V; ++e) v[e] = canon(u[0][e]);
+    const uint32_t nn = n0 + c, t4 = t0 + 8u * (V * j >> 2) + 4u * h + (V * j & 3u);
     if constexpr (GLU) {
         const bool odd = (lane & 1u) != 0u;
 #pragma unroll
-        for (int e = 0; e < 4; e += 2) {                           // every lane: the table is read by bpermute
-            const float a0 = dpp_f<kDppXor1>(v[e]), a1 = dpp_f<kDppXor1>(v[e + 1]);
-            const float hh = swiglu_reg(odd ? a1 : v[e], odd ? v[e + 1] : a0, a.ex, t64);
-            const uint32_t tt = t4 + (uint32_t)e + (odd ? 1u : 0u);
+        for (uint32_t e = 0; e < V; e += 2u) {                     // every lane: the table is read by bpermute
+            const float a0 = dpp_f<kDppXor1>(v[e]), a1 = dpp_f<kDppXor1>(v[e + 1u]);
+            const float hh = swiglu_reg(odd ? a1 : v[e], odd ? v[e + 1u] : a0, a.ex, t64);
+            const uint32_t tt = t4 + e + (odd ? 1u : 0u);
             if (tt < a.T && nn < a.N) a.y[(size_t)tt * a.y_stride + (nn >> 1)] = hh;
         }
     } else {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const uint32_t tt = t4 + (uint32_t)e;
+        for (uint32_t e = 0; e < V; ++e) {
+            const uint32_t tt = t4 + e;
             if (tt < a.T && nn < a.N) {
                 float y = v[e];
                 float * yp = a.y + (size_t)tt * a.y_stride + nn;
@@ -489,15 +500,29 @@ int tsr_launch_qact_mm4(const float * x, uint64_t x_stride, uint32_t K, uint32_t
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
-int tsr_launch_mm_q4_k(const tsr::MmArgs & a, hipStream_t s) {
+int tsr_launch_mm_q4_k(const tsr::MmArgs & a, uint32_t n_cu, hipStream_t s) {
     const tsr::WGeom g = tsr::wgeom(a.N, a.K >> 8, a.rb, true);
     if ((uint64_t)(31u / a.rb + 2u) * g.bstride >= 0x80000000ull) return -2;   // a tile's buffer window
     const uint32_t gx = (a.N + 31u) / 32u, gy = (a.T + 31u) / 32u;
     tsr::MmArgs m = a;
     m.grouped = (gx & 7u) == 0u && (uint64_t)a.N * (a.K / 256u) * 144u > (48ull << 20) ? 1u : 0u;   // measured
     const dim3 grid = m.grouped ? dim3(8u * gy, gx / 8u) : dim3(gx, gy);
-    if (a.glu) hipLaunchKernelGGL(tsr::k_mm_q4k<true>, grid, dim3(256), 0, s, m);
-    else hipLaunchKernelGGL(tsr::k_mm_q4k<false>, grid, dim3(256), 0, s, m);
+    // Eight waves a tile while the tiles leave the chip short of waves (one tile a CU; with long rows, two): the
+    // chain of a wave's super-blocks is then the time. With more tiles the eight-wave form's one workgroup a CU
+    // loses to three of four waves. Four -> eight waves, us: 2048x14336, 33 rows 22.8 -> 18.2, 128 rows (256 tiles)
+    // 26.0 -> 21.5, 256 rows (512) 37.1 -> 35.1, 512 rows (1024) 59.7 -> 62.8; 4096x4096, 64 rows 11.8 -> 11.0,
+    // 100 rows (512 tiles) 15.1 -> 16.2; 4096x2048, 64 rows 8.9 -> 8.3; rows of 4 super-blocks, which eight waves
+    // cannot share, 700x1024, 50 rows 6.8 -> 7.3.
+    const uint64_t tiles = (uint64_t)gx * gy;
+    const uint32_t nb = a.K >> 8;
+    const bool w8 = nb > 4u && (tiles <= n_cu || (tiles <= 2u * n_cu && nb >= 48u));
+    if (w8) {
+        if (a.glu) hipLaunchKernelGGL((tsr::k_mm_q4k<true, 8u>), grid, dim3(512), 0, s, m);
+        else hipLaunchKernelGGL((tsr::k_mm_q4k<false, 8u>), grid, dim3(512), 0, s, m);
+    } else {
+        if (a.glu) hipLaunchKernelGGL((tsr::k_mm_q4k<true, 4u>), grid, dim3(256), 0, s, m);
+        else hipLaunchKernelGGL((tsr::k_mm_q4k<false, 4u>), grid, dim3(256), 0, s, m);
+    }
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 

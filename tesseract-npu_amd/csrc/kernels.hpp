@@ -231,7 +231,7 @@ int tsr_launch_qact_mm(const float * x, uint64_t x_stride, uint32_t K, uint32_t 
 int tsr_launch_mm_q8_0(const tsr::MmArgs & a, hipStream_t s);
 int tsr_launch_qact_mm4(const float * x, uint64_t x_stride, uint32_t K, uint32_t T, uint32_t tp, uint8_t * xq,
                         uint32_t * xs, float * xd, hipStream_t s);
-int tsr_launch_mm_q4_k(const tsr::MmArgs & a, hipStream_t s);
+int tsr_launch_mm_q4_k(const tsr::MmArgs & a, uint32_t n_cu, hipStream_t s);
 // dst (device) <- bytes of pinned host memory, rounded up to 16, both 16-byte aligned (k_kv.hip)
 int tsr_launch_fetch(void * dst, const void * host, size_t bytes, hipStream_t s);
 int tsr_launch_kv_bytes(const tsr::KvArgs & a, uint32_t which, uint64_t off, uint64_t n, uint8_t * stage, int to_dev,

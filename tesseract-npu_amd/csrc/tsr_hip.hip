@@ -579,7 +579,7 @@ static int mul_mat_locked(tsr_hip_ctx * ctx, const tsr_hip_weight * w, const flo
             m.acc = a.acc;
             m.glu = a.glu;
             m.ex = a.ex;
-            if (tsr_launch_mm_q4_k(m, s)) return TSR_HIP_E_HIP;
+            if (tsr_launch_mm_q4_k(m, (uint32_t)ctx->n_cu, s)) return TSR_HIP_E_HIP;
         }
         return TSR_HIP_OK;
     }

@@ -209,3 +209,30 @@ def test_mm_q4_k_partial_counts(dev, oc, nsb):
     b[5, :, 4:] = 0xFF
     got, want = _mm(dev, oc, N, K, T, x=x, wblocks=blocks, fmt=1)
     assert_bits_equal(got, want, f"Q4_K {nsb} super-blocks")
+
+
+@pytest.mark.parametrize("N,nsb,T,glu", [
+    (8230, 9, 35, False),     # four waves: more tiles (516) than two a CU
+    (8230, 17, 35, True),
+    (8230, 49, 35, False),
+    (8228, 49, 20, False),    # eight waves: 258 tiles of long rows
+    (8228, 16, 20, True),     # the same tiles of shorter rows: four
+    (1030, 23, 35, True),     # eight waves: one tile a CU
+], ids=lambda v: str(v))
+def test_mm_q4_k_wave_counts(dev, oc, N, nsb, T, glu):
+    """The four- and eight-wave forms on both sides of the launcher's rule (256 CUs), with a token row whose
+    scale is below 2^-60 (spec operations)."""
+    K = 256 * nsb
+    x = S.normal(N + nsb, T * K).reshape(T, K)
+    x[3] *= np.float32(1e-22)
+    if not glu:
+        got, want = _mm(dev, oc, N, K, T, seed=nsb, x=x, add=True, fmt=1)
+    else:
+        blocks = weights(1, N, K, nsb)
+        full = oc.mul_mat(1, blocks, K, x, threads=8)
+        want = oc.swiglu(np.ascontiguousarray(full[:, 0::2]), np.ascontiguousarray(full[:, 1::2]))
+        w, yb = dev.weight(1, blocks, N, K), dev.alloc(4 * T * (N // 2))
+        dev.mul_mat(w, dev.upload(x), T, K, yb, N // 2, flags=tsr_hip.MM_GLU)
+        got = yb.read(np.float32, (T, N // 2))
+        w.free()
+    assert_bits_equal(got, want, f"Q4_K {N}x{K} T {T}")
