@@ -142,6 +142,29 @@ def test_fa_queued_work_lists(dev, oc, T, calls):
         assert_bits_equal(outs[i].read(np.float32, (T, nh * D)), want, f"call {i}")
 
 
+@pytest.mark.parametrize("T,n_head,n_head_kv,D", [(140, 20, 4, 128), (260, 6, 2, 256)], ids=["g5_d128", "g3_d256"])
+def test_fa_wide_merge(dev, oc, T, n_head, n_head_kv, D):
+    """More merge waves than the chip holds at once (256 CUs x 32): two values a lane, with head groups that do
+    not fill a workgroup and rows of one to more chunks than one round takes (4)."""
+    assert 4 * T * n_head_kv * ((n_head // n_head_kv + 3) // 4) * (D // 64) > 32 * 256
+    n, E = 9400, n_head_kv * D
+    kc, vc = _cache(oc, n, E, T)
+    q = S.normal(T + D, T * n_head * D).reshape(T, n_head * D)
+    hi = 1 + np.arange(T) % 37
+    hi[::29] = np.array([9400, 2050, 4100, 7000, 9300, 8300, 300, 2048, 6200])[:len(hi[::29])]
+    msum = np.zeros(8 + 4 * T, np.uint32)
+    msum[0], msum[1], msum[2] = 0x4D55534D, T, n
+    msum[9::4] = hi
+    scale = np.float32(1.0 / math.sqrt(D))
+    want = oc.flash_attn(q, kc, vc, D, n_head, n_head_kv, scale, msum, None, [])
+    K_, V_ = dev.kv(E, n), dev.kv(E, n)
+    K_.set_bytes(0, kc)
+    V_.set_bytes(1, vc)
+    out = dev.alloc(4 * T * n_head * D)
+    dev.flash_attn(dev.upload(q), T, n_head * D, K_, V_, D, n_head, n_head_kv, scale, msum, out, n_head * D)
+    assert_bits_equal(out.read(np.float32, (T, n_head * D)), want, f"{T} rows of {n_head} heads")
+
+
 def test_fa_general_and_two_run_masks(dev, oc):
     m2 = np.zeros((3, 100), np.float16); m2[:, 10:20] = -2.5; m2[1, 50:] = -np.inf
     got, want = _fa(dev, oc, 100, 112, 8, 2, 64, T=3, mask=m2)
