@@ -508,8 +508,9 @@ __global__ __launch_bounds__(256) void k_fa_qk(FaArgs a, FaPlan p) {
 
 // ---------------------------------------------------------------------------------------------
 // scores of many rows on the matrix cores: block (256-cell tile, 32 rows, query head), 4 waves of two 32-cell
-// subtiles. The rows' runs start at one cell, so their chunk cuts are multiples of 16 groups from there and
-// every row's 256-cell tiles are the same cells; the item of each (tile, row) comes from the host's map.
+// subtiles. The rows' runs start at one cell and their items on tile boundaries from there (the host's rule,
+// fa_score_tiles), so every row's 256-cell tiles are the same cells; the item of each (tile, row) comes from
+// the host's map.
 //
 // Per 32 rows x 32 cells and 32-value block, as in the prefill MUL_MAT: the integer block sums are one
 // v_mfma_i32_32x32x32_i8 (rows: queries, columns: cells) and the products dK Dx one

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "fa_item.hpp"
+
 namespace tsr {
 
 struct QactArgs {
@@ -90,18 +92,8 @@ struct KvArgs {
     uint32_t E, kv_size;
 };
 
-// One chunk of one query token (the planner's output), in execution order per token.
-struct FaItem {
-    uint32_t t;              // token
-    uint32_t u0, n;          // groups [u0, u0 + n)
-    uint32_t c_lo, c_hi;     // visible chunk-relative cells (FAST)
-    uint32_t general;        // GENERAL chunk: all cells, f32 mask added
-    uint32_t s_off;          // first score cell of the item in S (scores at S + s_off * n_head)
-    uint32_t tile0, ntiles;  // its 256-cell score tiles (rows tile0 .. tile0 + ntiles - 1 of Mpart)
-};
 // The work list of one call. Small lists (decode) travel inline in the kernel arguments; larger ones
 // are copied to device memory once per call and the kernels read them there (FaArgs::items != 0).
-constexpr uint32_t kFaInlItems = 48, kFaInlTok = 8;
 struct FaPlan {
     uint32_t n_items, maxtiles;                        // items; tiles of the largest item
     uint32_t tok_first[kFaInlTok], tok_count[kFaInlTok];

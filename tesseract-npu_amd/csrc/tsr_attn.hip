@@ -11,6 +11,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "fa_plan.hpp"
 #include "kernels.hpp"
 #include "runtime.hpp"
 #include "tsr_hip.h"
@@ -241,97 +242,6 @@ int tsr_hip_msum_mask_f32(const uint16_t * mask, size_t row_stride, uint32_t n_k
 // ---------------------------------------------------------------------------------------------
 namespace {
 
-constexpr uint32_t kC = 4u, kPcap = 9344u;
-
-struct Chunk {
-    uint32_t u0, n, c_lo, c_hi, general;
-};
-
-// NCG = min(128, C floor(PCAP / (16 E / D)), max(4C, roundup_4C(ceil(n_total / 2))))
-// (sw/sim/include/tsr_fa_plan.h:130-156).
-uint32_t ncg_of(uint32_t E, uint32_t D, uint32_t n_total) {
-    const uint64_t pc = (uint64_t)kC * (kPcap / (16u * (E / D)));
-    const uint64_t half = ((uint64_t)n_total + 1u) / 2u, c4 = 4u * kC;
-    const uint64_t m = half <= c4 ? c4 : (half + c4 - 1u) / c4 * c4;
-    return (uint32_t)std::min<uint64_t>(std::min<uint64_t>(128u, pc), m);
-}
-
-// The chunks of one query row in execution order (one-row tiles: rules 1, 2, 4, 7, 8 of the planner,
-// sw/sim/include/tsr_fa_plan.h:16-42). Returns false for a malformed MSUM row.
-// A fixed-capacity stand-in for std::vector in the planner of the entry point that allocates nothing:
-// push_back past the capacity records an overflow instead of growing.
-template <class T, size_t N>
-struct FixedVec {
-    T v[N];
-    size_t n = 0;
-    bool overflow = false;
-    void clear() { n = 0; overflow = false; }
-    void push_back(const T & x) {
-        if (n < N) v[n++] = x;
-        else overflow = true;
-    }
-    void assign(size_t k, const T & x) {
-        if (k > N) { overflow = true; k = N; }
-        n = k;
-        for (size_t i = 0; i < k; ++i) v[i] = x;
-    }
-    size_t size() const { return n; }
-    T & operator[](size_t i) { return v[i]; }
-    const T & operator[](size_t i) const { return v[i]; }
-    T * data() { return v; }
-    const T * begin() const { return v; }
-    const T * end() const { return v + n; }
-};
-template <class V> bool overflowed(const V &) { return false; }
-template <class T, size_t N> bool overflowed(const FixedVec<T, N> & v) { return v.overflow; }
-
-template <class Out>
-bool plan_row(uint32_t E, uint32_t D, const uint32_t * words, uint32_t q, const uint32_t (*new_runs)[2],
-              uint32_t n_new, Out & out) {
-    const uint32_t n_kv = words[2];
-    const bool general = (words[3] & 1u) != 0u;
-    struct Sub { uint32_t ulo, uhi; uint64_t lo, hi; } sub[2];
-    uint32_t nsub = 0;
-    if (general) {
-        if (n_kv > 0u) sub[nsub++] = { 0u, (n_kv + 15u) / 16u, 0u, 0u };
-    } else {
-        const uint32_t * w = words + 8u + 4u * q;
-        if (w[0] > w[1] || w[2] > w[3] || w[1] > n_kv || w[3] > n_kv) return false;
-        if (w[1] > w[0] && w[3] > w[2] && !(w[1] <= w[2] || w[3] <= w[0])) return false;
-        uint32_t r[2][2], nr = 0;
-        if (w[1] > w[0]) { r[nr][0] = w[0]; r[nr][1] = w[1]; ++nr; }
-        if (w[3] > w[2]) { r[nr][0] = w[2]; r[nr][1] = w[3]; ++nr; }
-        if (nr == 2u && r[1][0] < r[0][0]) { std::swap(r[0][0], r[1][0]); std::swap(r[0][1], r[1][1]); }
-        for (uint32_t k = 0; k < nr; ++k) sub[nsub++] = { r[k][0] / 16u, (r[k][1] + 15u) / 16u, r[k][0], r[k][1] };
-    }
-    if (nsub == 0u) {                                      // no visible cell: one empty chunk
-        out.push_back({ 0u, 1u, 0u, 0u, 0u });
-        return true;
-    }
-    uint32_t n_total = 0;
-    for (uint32_t k = 0; k < nsub; ++k) n_total += sub[k].uhi - sub[k].ulo;
-    const uint32_t ncg = ncg_of(E, D, n_total);
-    if (ncg == 0u) return false;
-    for (int pass = 0; pass < 2; ++pass)                   // chunks holding a new cell go last
-        for (uint32_t k = 0; k < nsub; ++k)
-            for (uint32_t a = sub[k].ulo; a < sub[k].uhi; a += ncg) {
-                const uint32_t b = std::min(a + ncg, sub[k].uhi);
-                bool has_new = false;
-                for (uint32_t i = 0; i < n_new; ++i)
-                    has_new |= new_runs[i][1] > new_runs[i][0] && (uint64_t)new_runs[i][0] < 16ull * b &&
-                                (uint64_t)new_runs[i][1] > 16ull * a;
-                if ((int)has_new != pass) continue;
-                Chunk c{ a, b - a, 0u, 16u * (b - a), general ? 1u : 0u };
-                if (!general) {
-                    const int64_t A = 16 * (int64_t)a, n16 = 16 * (int64_t)(b - a);
-                    c.c_lo = (uint32_t)std::max<int64_t>((int64_t)sub[k].lo - A, 0);
-                    c.c_hi = (uint32_t)std::min<int64_t>((int64_t)sub[k].hi - A, n16);
-                }
-                out.push_back(c);
-            }
-    return true;
-}
-
 size_t up256(size_t x) { return (x + 255u) & ~(size_t)255u; }
 
 // The shape checks FLASH_ATTN_EXT makes on its operands (the planned and the unplanned entry points).
@@ -343,62 +253,6 @@ int fa_check_shape(uint32_t D, uint32_t n_head, uint32_t n_head_kv, float scale)
     uint32_t sb;
     memcpy(&sb, &scale, 4);
     if ((sb >> 31) || (sb & 0x7F800000u) == 0u || (sb & 0x7F800000u) == 0x7F800000u) return TSR_HIP_E_SHAPE;
-    return TSR_HIP_OK;
-}
-
-// The work list of one call: every token row planned, flattened into items (chunks) with their
-// 256-cell score tiles; tok = tok_first[T] | tok_count[T]. FaWorkFixed holds at most the inline list
-// (kFaInlItems items of at most kFaInlTok tokens) in fixed arrays: planning it allocates nothing.
-template <class Items, class Tok, class Chunks>
-struct FaWorkT {
-    Items items;
-    Tok tok;
-    Chunks ch;               // one row's chunks (planner temporary)
-    uint64_t cells = 0;
-    uint32_t n_tiles = 0, maxtiles = 1, max_groups = 0;
-};
-using FaWork = FaWorkT<std::vector<tsr::FaItem>, std::vector<uint32_t>, std::vector<Chunk>>;
-using FaWorkFixed = FaWorkT<FixedVec<tsr::FaItem, tsr::kFaInlItems>, FixedVec<uint32_t, 2u * tsr::kFaInlTok>,
-                            FixedVec<Chunk, tsr::kFaInlItems>>;
-
-// Returns TSR_HIP_E_RANGE when a fixed-capacity work list overflows.
-template <class W>
-int fa_plan_rows(uint32_t E, uint32_t D, uint32_t T, const uint32_t * msum, const uint32_t (*new_runs)[2], uint32_t n_new,
-                 bool have_mask, W & w) {
-    w.items.clear();
-    w.tok.assign(2u * (size_t)T, 0u);
-    if (overflowed(w.tok)) return TSR_HIP_E_RANGE;
-    w.cells = 0;
-    w.n_tiles = 0;
-    w.maxtiles = 1;
-    w.max_groups = 0;
-    auto & ch = w.ch;
-    for (uint32_t t = 0; t < T; ++t) {
-        ch.clear();
-        if (!plan_row(E, D, msum, t, new_runs, n_new, ch)) return TSR_HIP_E_MASK;
-        if (overflowed(ch)) return TSR_HIP_E_RANGE;
-        w.tok[t] = (uint32_t)w.items.size();
-        w.tok[T + t] = (uint32_t)ch.size();
-        for (const Chunk & c : ch) {
-            if (c.general && !have_mask) return TSR_HIP_E_MASK;
-            tsr::FaItem it{};
-            it.t = t;
-            it.u0 = c.u0;
-            it.n = c.n;
-            it.c_lo = c.c_lo;
-            it.c_hi = c.c_hi;
-            it.general = c.general;
-            it.s_off = (uint32_t)w.cells;
-            it.tile0 = w.n_tiles;
-            it.ntiles = (16u * c.n + 255u) / 256u;
-            w.n_tiles += it.ntiles;
-            w.maxtiles = std::max(w.maxtiles, it.ntiles);
-            w.max_groups = std::max(w.max_groups, c.n);
-            w.cells += 16u * c.n;
-            w.items.push_back(it);
-        }
-        if (overflowed(w.items)) return TSR_HIP_E_RANGE;
-    }
     return TSR_HIP_OK;
 }
 
@@ -448,39 +302,24 @@ static int fa_unplanned(tsr_hip_ctx * ctx, const float * q_dev, uint32_t T, uint
         return TSR_HIP_E_ARG;
     if (NOALLOC && T > tsr::kFaInlTok) return TSR_HIP_E_RANGE;
 
-    typename std::conditional<NOALLOC, FaWorkFixed, FaWork>::type w;
-    if ((rc = fa_plan_rows(E, D, T, msum, new_runs, n_new, mask_f32_dev != nullptr, w)) != 0) return rc;
+    typename std::conditional<NOALLOC, tsr::FaWorkFixed, tsr::FaWork>::type w;
+    if ((rc = tsr::fa_plan_rows(E, D, T, msum, new_runs, n_new, mask_f32_dev != nullptr, w)) != 0) return rc;
     const size_t n_items = w.items.size();
     if (w.cells * n_head > 0xFFFFFFFFull || n_items * 4u > 0x7FFFFFFFull || n_items * w.maxtiles > 0x7FFFFFFFull)
         return TSR_HIP_E_SHAPE;
     const bool inl = n_items <= tsr::kFaInlItems && T <= tsr::kFaInlTok;
-    // The scores of many rows on the matrix cores (k_fa_qk_mm): one FAST run per row, all from one cell, so
-    // that the rows' chunk cuts (multiples of 16 groups) fall on common 256-cell tiles. It needs the queries'
-    // quantization as a launch of its own (3-6 us), and pays from ~4 M scores of D 128 on. Measured, one-row
-    // kernel -> QACT + this one: 512 rows behind 1536 cells (29 M scores) 110 -> 56 us, 300 rows behind 700
-    // (8 M) 38 -> 30, D 64: 256 rows from cell 0 (1.3 M) 9.4 -> 13.7.
-    uint32_t n_map = 0, lo = 0;
-    if constexpr (!NOALLOC) {
-        bool uni = !inl && D <= 128u && (msum[3] & 1u) == 0u && w.cells * n_head * (D / 64u) >= (10ull << 20) &&
-                   4u * w.cells * n_head < (1ull << 31) && (uint64_t)T * K < (1ull << 31);
-        lo = msum[8];
-        for (uint32_t t = 0; uni && t < T; ++t) {
-            const uint32_t * r = msum + 8u + 4u * t;
-            uni = r[0] == lo && r[1] > r[0] && r[2] >= r[3];
-            n_map = std::max(n_map, ((r[1] + 15u) / 16u - lo / 16u + 15u) / 16u);
-        }
-        if (!uni) n_map = 0;
-    }
+    uint32_t n_map = 0, lo = 0;                                   // scores on the matrix cores
+    if constexpr (!NOALLOC)
+        if (!inl) n_map = tsr::fa_score_tiles(w, D, n_head, T, msum, lo);
     size_t off = 0;
-    const size_t map_words = n_map ? (size_t)n_map * T + T : 0u;  // the tile map and the rows' run ends
-    const size_t o_items = off;
-    off = up256(off + (inl ? 0u : n_items * sizeof(tsr::FaItem) + 8u * (size_t)T + 4u * map_words));
+    const size_t list_bytes = tsr::fa_list_bytes(n_items, T, n_map);
+    const size_t o_items = off; off = up256(off + (inl ? 0u : list_bytes));
     const size_t o_xq = off; off = up256(off + (n_map ? (size_t)T * K : 0u));
     const size_t o_xd = off; off = up256(off + (n_map ? (size_t)T * K / 8u : 0u));
     const size_t o_S = off; off = up256(off + 4u * (size_t)w.cells * n_head);
     const size_t o_Mp = off; off = up256(off + 4u * (size_t)w.n_tiles * n_head);
-    const size_t o_OP = off; off = up256(off + 4u * n_items * kC * n_head * D);
-    const size_t o_LP = off; off = up256(off + 4u * n_items * kC * n_head);
+    const size_t o_OP = off; off = up256(off + 4u * n_items * tsr::kC * n_head * D);
+    const size_t o_LP = off; off = up256(off + 4u * n_items * tsr::kC * n_head);
     if (NOALLOC && off > kFaNoAllocBytes) return TSR_HIP_E_RANGE;
 
     tsr::FaPlan p{};
@@ -490,20 +329,6 @@ static int fa_unplanned(tsr_hip_ctx * ctx, const float * q_dev, uint32_t T, uint
         std::copy(w.items.begin(), w.items.end(), p.items);
         for (uint32_t t = 0; t < T; ++t) { p.tok_first[t] = w.tok[t]; p.tok_count[t] = w.tok[T + t]; }
     }
-    // items | tok_first | tok_count (| tile map | run ends)
-    const size_t list_bytes = n_items * sizeof(tsr::FaItem) + 8u * (size_t)T + 4u * map_words;
-    auto pack = [&](uint8_t * list) {
-        memcpy(list, w.items.data(), n_items * sizeof(tsr::FaItem));
-        memcpy(list + n_items * sizeof(tsr::FaItem), w.tok.data(), 8u * (size_t)T);
-        if (n_map == 0u) return;
-        uint32_t * m = (uint32_t *)(list + n_items * sizeof(tsr::FaItem) + 8u * (size_t)T);
-        std::fill(m, m + (size_t)n_map * T, 0xFFFFFFFFu);
-        for (size_t i = 0; i < n_items; ++i) {
-            const tsr::FaItem & it = w.items[i];
-            for (uint32_t k = 0, a0 = (it.u0 - lo / 16u) / 16u; k < it.ntiles; ++k) m[(size_t)(a0 + k) * T + it.t] = (uint32_t)i;
-        }
-        for (uint32_t t = 0; t < T; ++t) m[(size_t)n_map * T + t] = msum[8u + 4u * t + 1u];
-    };
 
     std::lock_guard<std::mutex> lk(ctx->mtx);
     (void)hipSetDevice(ctx->device);
@@ -521,11 +346,11 @@ static int fa_unplanned(tsr_hip_ctx * ctx, const float * q_dev, uint32_t T, uint
             // when the graph replays): long work lists are for eager calls or a tsr_hip_fa_plan
             if (tsr_capturing(s)) return TSR_HIP_E_ARG;
             if (uint8_t * slot = ctx->lists.acquire(list_bytes)) {
-                pack(slot);
+                tsr::fa_pack_list(w, T, n_map, lo, msum, slot);
                 rc = ctx->lists.send(base + o_items, list_bytes, s);
             } else {
                 std::vector<uint8_t> packed(list_bytes);
-                pack(packed.data());
+                tsr::fa_pack_list(w, T, n_map, lo, msum, packed.data());
                 rc = hip_err(hipMemcpyAsync(base + o_items, packed.data(), list_bytes, hipMemcpyHostToDevice, s), "fa plan");
             }
             if (rc) return rc;
@@ -622,8 +447,8 @@ int tsr_hip_fa_plan_create(tsr_hip_ctx * ctx, uint32_t D, uint32_t n_head, uint3
     if (rc) return rc;
     if (T > 65535u) return TSR_HIP_E_SHAPE;
     const uint32_t E = n_head_kv * D;
-    const uint64_t pc = (uint64_t)kC * (kPcap / (16u * (E / D)));
-    const uint64_t ncg_min = std::max<uint64_t>(1u, std::min<uint64_t>(std::min<uint64_t>(128u, pc), 4u * kC));
+    const uint64_t pc = (uint64_t)tsr::kC * (tsr::kPcap / (16u * (E / D)));
+    const uint64_t ncg_min = std::max<uint64_t>(1u, std::min<uint64_t>(std::min<uint64_t>(128u, pc), 4u * tsr::kC));
     const uint64_t groups = ((uint64_t)kv_size + 15u) / 16u + 2u;             // two runs, each with a partial group
     const uint64_t items = (uint64_t)T * ((groups + ncg_min - 1u) / ncg_min + 2u);
     const uint64_t cells = (uint64_t)T * 16u * groups;
@@ -643,13 +468,13 @@ int tsr_hip_fa_plan_create(tsr_hip_ctx * ctx, uint32_t D, uint32_t n_head, uint3
     p->o_items = off; off = up256(off + items * sizeof(tsr::FaItem) + 8u * (size_t)T);
     p->o_S = off; off = up256(off + 4u * (size_t)cells * n_head);
     p->o_Mp = off; off = up256(off + 4u * (size_t)tiles * n_head);
-    p->o_OP = off; off = up256(off + 4u * (size_t)items * kC * n_head * D);
-    p->o_LP = off; off = up256(off + 4u * (size_t)items * kC * n_head);
+    p->o_OP = off; off = up256(off + 4u * (size_t)items * tsr::kC * n_head * D);
+    p->o_LP = off; off = up256(off + 4u * (size_t)items * tsr::kC * n_head);
     // the fused decode form (T == 1): per-tile segment results and row sums, and its counters
     const uint64_t ftiles = T == 1u ? tiles : 0u;
     // (value, tag) pairs of the decode form: segment results, row sums, chunk maxima
-    p->o_SO = off; off = up256(off + 8u * (size_t)ftiles * kC * n_head * D);
-    p->o_SL = off; off = up256(off + 8u * (size_t)ftiles * kC * n_head);
+    p->o_SO = off; off = up256(off + 8u * (size_t)ftiles * tsr::kC * n_head * D);
+    p->o_SL = off; off = up256(off + 8u * (size_t)ftiles * tsr::kC * n_head);
     p->o_MI = off; off = up256(off + (T == 1u ? 8u * (size_t)items * n_head : 0u));
     // zero between launches: the 16-byte slots of segment maxima (an item has <= 8 tiles of 4 channels:
     // NCG <= 128 groups) and the counters
@@ -710,8 +535,8 @@ int tsr_hip_fa_plan_set(tsr_hip_ctx * ctx, tsr_hip_fa_plan * plan, const uint32_
                         const uint32_t (*new_runs)[2], uint32_t n_new, int * shape_changed, void * stream) {
     if (ctx == nullptr || plan == nullptr || msum == nullptr || (n_new && new_runs == nullptr)) return TSR_HIP_E_ARG;
     if (msum[0] != 0x4D55534Du || msum[1] != plan->T || msum[2] > plan->kv_size) return TSR_HIP_E_MASK;
-    FaWork w;
-    int rc = fa_plan_rows(plan->n_head_kv * plan->D, plan->D, plan->T, msum, new_runs, n_new, mask_f32 != 0, w);
+    tsr::FaWork w;
+    int rc = tsr::fa_plan_rows(plan->n_head_kv * plan->D, plan->D, plan->T, msum, new_runs, n_new, mask_f32 != 0, w);
     if (rc) return rc;
     if (w.items.size() > plan->items_max || w.cells > plan->cells_max || w.n_tiles > plan->tiles_max)
         return TSR_HIP_E_SHAPE;

@@ -119,6 +119,34 @@ def test_fa_rows_matrix_core_scores(dev, oc, T, lo, hist, n_head, n_head_kv, D, 
     assert_bits_equal(out.read(np.float32, (T, n_head * D)), want, f"{T} rows behind {hist}")
 
 
+@pytest.mark.parametrize("T,hist,n_head,n_head_kv,D", [
+    (64, 2560, 32, 32, 128),   # chunks of 72 groups: no multiple of a tile
+    (52, 2500, 40, 40, 128),   # 56
+    (128, 2600, 32, 32, 64),   # 72
+    (66, 4200, 20, 20, 128),   # 116
+    (70, 3900, 24, 24, 128),   # 96: several chunks a row on tile boundaries
+], ids=["kv32", "kv40", "kv32_d64", "kv20", "kv24"])
+def test_fa_rows_many_kv_heads(dev, oc, T, hist, n_head, n_head_kv, D):
+    """Many rows of several chunks whose length follows from the number of KV heads, with enough scores for the
+    matrix-core score kernel: it may run only where the chunk cuts fall on its 256-cell tiles."""
+    n, E = hist + T, n_head_kv * D
+    assert sum((hist + t + 16) // 16 * 16 for t in range(T)) * n_head * (D // 64) >= 10 << 20
+    kc, vc = _cache(oc, n, E, T + D)
+    q = S.normal(T, T * n_head * D).reshape(T, n_head * D)
+    msum = np.zeros(8 + 4 * T, np.uint32)
+    msum[0], msum[1], msum[2] = 0x4D55534D, T, n
+    msum[9::4] = hist + 1 + np.arange(T)
+    scale = np.float32(1.0 / math.sqrt(D))
+    want = oc.flash_attn(q, kc, vc, D, n_head, n_head_kv, scale, msum, None, [[hist, n]])
+    K_, V_ = dev.kv(E, n), dev.kv(E, n)
+    K_.set_bytes(0, kc)
+    V_.set_bytes(1, vc)
+    out = dev.alloc(4 * T * n_head * D)
+    dev.flash_attn(dev.upload(q), T, n_head * D, K_, V_, D, n_head, n_head_kv, scale, msum, out, n_head * D,
+                   new_runs=[[hist, n]])
+    assert_bits_equal(out.read(np.float32, (T, n_head * D)), want, f"{T} rows of {n_head_kv} KV heads")
+
+
 @pytest.mark.parametrize("T,calls", [(40, 11), (7000, 2)], ids=["slots_reused", "list_beyond_a_slot"])
 def test_fa_queued_work_lists(dev, oc, T, calls):
     """Unplanned calls with work lists of their own queued behind each other without a wait: each sees its own
