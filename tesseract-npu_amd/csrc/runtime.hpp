@@ -102,7 +102,10 @@ struct tsr_staging {
         uint8_t * slot = host + (size_t)k * kSlotBytes;
         memcpy(slot, src, bytes);
         int rc = tsr::hip_err(hipMemcpyAsync(dst_dev, slot, bytes, hipMemcpyHostToDevice, s), "hipMemcpyAsync staging");
-        if (rc == 0) rc = tsr::hip_err(hipEventRecord(ev[k], s), "hipEventRecord staging");
+        if (rc == 0) {
+            rc = tsr::hip_err(hipEventRecord(ev[k], s), "hipEventRecord staging");
+            if (rc) (void)hipStreamSynchronize(s);                // no event: the copy has run before the slot is free
+        }
         used[k] = rc == 0;
         return rc;
     }
@@ -153,6 +156,7 @@ struct tsr_lists {
         next = (next + 1u) % kSlots;
         if (tsr_launch_fetch(dst_dev, host + k * kSlotBytes, bytes, s)) return TSR_HIP_E_HIP;
         const int rc = tsr::hip_err(hipEventRecord(ev[k], s), "hipEventRecord list");
+        if (rc) (void)hipStreamSynchronize(s);                    // no event: the kernel has run before the slot is free
         used[k] = rc == 0;
         return rc;
     }
