@@ -206,4 +206,28 @@ void fa_pack_list(const W & w, uint32_t T, uint32_t n_map, uint32_t lo, const ui
     for (uint32_t t = 0; t < T; ++t) m[(size_t)n_map * T + t] = msum[8u + 4u * t + 1u];
 }
 
+// The scratch of one unplanned call (byte offsets). With n_map != 0 the tail of the list (tile map, run ends) and
+// the quantized queries lie where the P.V kernel later writes the channel partials: the score kernel, which runs
+// before it, is their only reader, and the call needs no more scratch than on the other route.
+struct FaLayout {
+    size_t S, Mp, LP, items, OP, xq, xd, bytes;
+};
+inline FaLayout fa_layout(size_t n_items, uint64_t cells, uint32_t n_tiles, uint32_t T, uint32_t n_head, uint32_t D,
+                          bool inl, uint32_t n_map) {
+    auto up256 = [](size_t x) { return (x + 255u) & ~(size_t)255u; };
+    const size_t K = (size_t)n_head * D;
+    FaLayout l{};
+    l.Mp = up256(4u * (size_t)cells * n_head);
+    l.LP = l.Mp + up256(4u * (size_t)n_tiles * n_head);
+    l.items = l.LP + up256(4u * n_items * kC * n_head);
+    l.OP = l.items + (inl ? 0u : up256(fa_list_bytes(n_items, T, 0u)));
+    l.bytes = l.OP + up256(4u * n_items * kC * K);
+    if (n_map != 0u) {
+        l.xq = up256(l.items + fa_list_bytes(n_items, T, n_map));
+        l.xd = l.xq + up256(T * K);
+        l.bytes = std::max(l.bytes, l.xd + up256(T * K / 8u));
+    }
+    return l;
+}
+
 }  // namespace tsr

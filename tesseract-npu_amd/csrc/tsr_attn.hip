@@ -311,16 +311,9 @@ static int fa_unplanned(tsr_hip_ctx * ctx, const float * q_dev, uint32_t T, uint
     uint32_t n_map = 0, lo = 0;                                   // scores on the matrix cores
     if constexpr (!NOALLOC)
         if (!inl) n_map = tsr::fa_score_tiles(w, D, n_head, T, msum, lo);
-    size_t off = 0;
     const size_t list_bytes = tsr::fa_list_bytes(n_items, T, n_map);
-    const size_t o_items = off; off = up256(off + (inl ? 0u : list_bytes));
-    const size_t o_xq = off; off = up256(off + (n_map ? (size_t)T * K : 0u));
-    const size_t o_xd = off; off = up256(off + (n_map ? (size_t)T * K / 8u : 0u));
-    const size_t o_S = off; off = up256(off + 4u * (size_t)w.cells * n_head);
-    const size_t o_Mp = off; off = up256(off + 4u * (size_t)w.n_tiles * n_head);
-    const size_t o_OP = off; off = up256(off + 4u * n_items * tsr::kC * n_head * D);
-    const size_t o_LP = off; off = up256(off + 4u * n_items * tsr::kC * n_head);
-    if (NOALLOC && off > kFaNoAllocBytes) return TSR_HIP_E_RANGE;
+    const tsr::FaLayout lay = tsr::fa_layout(n_items, w.cells, w.n_tiles, T, n_head, D, inl, n_map);
+    if (NOALLOC && lay.bytes > kFaNoAllocBytes) return TSR_HIP_E_RANGE;
 
     tsr::FaPlan p{};
     p.n_items = (uint32_t)n_items;
@@ -338,7 +331,7 @@ static int fa_unplanned(tsr_hip_ctx * ctx, const float * q_dev, uint32_t T, uint
         if (ctx->fa_fixed == nullptr) return TSR_HIP_E_HIP;       // the array's address was not found at open
         base = ctx->fa_fixed;
     } else {
-        rc = ctx->scratch.reserve(off, s);
+        rc = ctx->scratch.reserve(lay.bytes, s);
         if (rc) return rc;
         base = (uint8_t *)ctx->scratch.ptr;
         if (!inl) {
@@ -347,11 +340,11 @@ static int fa_unplanned(tsr_hip_ctx * ctx, const float * q_dev, uint32_t T, uint
             if (tsr_capturing(s)) return TSR_HIP_E_ARG;
             if (uint8_t * slot = ctx->lists.acquire(list_bytes)) {
                 tsr::fa_pack_list(w, T, n_map, lo, msum, slot);
-                rc = ctx->lists.send(base + o_items, list_bytes, s);
+                rc = ctx->lists.send(base + lay.items, list_bytes, s);
             } else {
                 std::vector<uint8_t> packed(list_bytes);
                 tsr::fa_pack_list(w, T, n_map, lo, msum, packed.data());
-                rc = hip_err(hipMemcpyAsync(base + o_items, packed.data(), list_bytes, hipMemcpyHostToDevice, s), "fa plan");
+                rc = hip_err(hipMemcpyAsync(base + lay.items, packed.data(), list_bytes, hipMemcpyHostToDevice, s), "fa plan");
             }
             if (rc) return rc;
         }
@@ -359,14 +352,14 @@ static int fa_unplanned(tsr_hip_ctx * ctx, const float * q_dev, uint32_t T, uint
     tsr::FaArgs a = fa_args(ctx, q_dev, q_stride, kc, vc, D, n_head, n_head_kv, scale, mask_f32_dev,
                             16u * ((msum[2] + 15u) / 16u), out_dev, out_stride);
     if (!inl) {
-        a.items = (const tsr::FaItem *)(base + o_items);
-        a.tok_first = (const uint32_t *)(base + o_items + n_items * sizeof(tsr::FaItem));
+        a.items = (const tsr::FaItem *)(base + lay.items);
+        a.tok_first = (const uint32_t *)(base + lay.items + n_items * sizeof(tsr::FaItem));
         a.tok_count = a.tok_first + T;
     }
-    a.S = (float *)(base + o_S);
-    a.Mpart = (float *)(base + o_Mp);
-    a.OP = (float *)(base + o_OP);
-    a.LP = (float *)(base + o_LP);
+    a.S = (float *)(base + lay.S);
+    a.Mpart = (float *)(base + lay.Mp);
+    a.OP = (float *)(base + lay.OP);
+    a.LP = (float *)(base + lay.LP);
     a.max_groups = w.max_groups;
     if (n_map != 0u) {
         a.tmap = a.tok_count + T;
@@ -374,10 +367,10 @@ static int fa_unplanned(tsr_hip_ctx * ctx, const float * q_dev, uint32_t T, uint
         a.n_map = n_map;
         a.u_lo = lo / 16u;
         a.lo = lo;
-        a.xq = base + o_xq;
-        a.xd = (const float *)(base + o_xd);
+        a.xq = base + lay.xq;
+        a.xd = (const float *)(base + lay.xd);
         a.s_bytes = (uint32_t)(4u * w.cells * n_head);
-        if (tsr_launch_qact_mm(q_dev, q_stride, K, T, base + o_xq, (float *)(base + o_xd), s)) return TSR_HIP_E_HIP;
+        if (tsr_launch_qact_mm(q_dev, q_stride, K, T, base + lay.xq, (float *)(base + lay.xd), s)) return TSR_HIP_E_HIP;
     }
     ctx->ctr.flash_attn_calls++;
     ctx->ctr.flash_attn_kv_bytes += w.cells * (uint64_t)E / 32u * 34u * 2u;

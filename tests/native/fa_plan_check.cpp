@@ -37,6 +37,28 @@ static const char * check(const FaWork & w, uint32_t T, uint32_t n_head, uint32_
     return nullptr;
 }
 
+// The scratch: no more than the other route's, and nothing that is alive together overlaps.
+static const char * check_layout(const FaWork & w, uint32_t T, uint32_t n_head, uint32_t D, uint32_t n_map) {
+    const size_t n = w.items.size(), K = (size_t)n_head * D;
+    const FaLayout l = fa_layout(n, w.cells, w.n_tiles, T, n_head, D, false, n_map);
+    if (l.bytes > fa_layout(n, w.cells, w.n_tiles, T, n_head, D, false, 0u).bytes) return "more scratch than the one-row route";
+    struct Part { size_t at, bytes; };
+    const Part S = { l.S, 4u * (size_t)w.cells * n_head }, Mp = { l.Mp, 4u * (size_t)w.n_tiles * n_head },
+               LP = { l.LP, 16u * n * n_head }, OP = { l.OP, 16u * n * K }, items = { l.items, fa_list_bytes(n, T, 0u) },
+               list = { l.items, (fa_list_bytes(n, T, n_map) + 15u) / 16u * 16u }, xq = { l.xq, T * K }, xd = { l.xd, T * K / 8u };
+    auto apart = [&](std::vector<Part> p) {
+        for (size_t i = 0; i < p.size(); ++i) {
+            if (p[i].at % 256u != 0u || p[i].at + p[i].bytes > l.bytes) return false;
+            for (size_t j = 0; j < i; ++j)
+                if (p[i].at < p[j].at + p[j].bytes && p[j].at < p[i].at + p[i].bytes) return false;
+        }
+        return true;
+    };
+    std::vector<Part> scores = { S, Mp, list }, rest = { S, Mp, LP, OP, items };   // up to the scores; from P.V on
+    if (n_map != 0u) scores.insert(scores.end(), { xq, xd });
+    return apart(scores) && apart(rest) ? nullptr : "overlapping scratch";
+}
+
 int main() {
     size_t taken = 0, refused = 0, cut = 0;
     for (uint32_t nkv = 1; nkv <= 64; ++nkv)
@@ -66,6 +88,7 @@ int main() {
                             }
                             const bool enough = w.cells * n_head * (D / 64u) >= (10ull << 20) && 4u * w.cells * n_head < (1ull << 31);
                             const char * bad = n_map ? check(w, T, n_head, n_map, first, msum.data()) : nullptr;
+                            if (bad == nullptr) bad = check_layout(w, T, n_head, D, n_map);
                             if (bad == nullptr && (n_map != 0u) != (aligned && enough)) bad = "the route's rule";
                             if (bad != nullptr) {
                                 printf("%s: %u of %u heads, D %u, %u rows behind %u cells from %u\n", bad, nkv, n_head, D, T, hist, lo);
