@@ -162,25 +162,36 @@ int fa_plan_rows(uint32_t E, uint32_t D, uint32_t T, const uint32_t * msum, cons
 
 // The scores of many rows on the matrix cores (k_fa_qk_mm), or 0: the one-row kernel (k_fa_qk). Returns the
 // number of 256-cell score tiles from group lo / 16 on and in lo the first visible cell of the rows.
-// One FAST run per row, all from one cell, and every item on a tile boundary from there: a tile then lies in
-// one item of each row. The chunk cuts are on such boundaries while NCG is a multiple of 16 groups, which the
-// planner's cap of 4 floor(9344 / (16 n_head_kv)) is not for every n_head_kv (72 groups for 32 KV heads, 116
-// for 20), so the items themselves are looked at. It needs the queries' quantization as a launch of its own
-// (3-6 us), and pays from ~4 M scores of D 128 on. Measured, one-row kernel -> QACT + this one: 512 rows
-// behind 1536 cells (29 M scores) 110 -> 56 us, 300 rows behind 700 (8 M) 38 -> 30, D 64: 256 rows from cell 0
-// (1.3 M) 9.4 -> 13.7.
+// - One FAST run per row, all from one cell, and every item on a tile boundary from there: a tile then lies in
+//   one item of each row. The chunk cuts are on such boundaries while NCG is a multiple of 16 groups, which the
+//   planner's cap of 4 floor(9344 / (16 n_head_kv)) is not for every n_head_kv (72 groups for 32 KV heads, 116
+//   for 20), so the items themselves are looked at.
+// - Enough scores: it needs the queries' quantization as a launch of its own (3-6 us), and pays from ~4 M scores
+//   of D 128 on. Measured, one-row kernel -> QACT + this one: 512 rows behind 1536 cells (29 M scores) 110 -> 56
+//   us, 300 rows behind 700 (8 M) 38 -> 30, D 64: 256 rows from cell 0 (1.3 M) 9.4 -> 13.7.
+// - At least two thirds of the scores that it forms in use: a workgroup forms a tile for 32 rows when one of them
+//   reaches it. Whole calls, one-row kernel -> this one, 64 query heads of D 128: 1 row of 103 K cells 115 ->
+//   407 us, 8 rows of 22 K 123 -> 162, 512 rows, 16 of them of 6000 cells and the others of 40, 365 -> 582; behind
+//   12 K cells 17 rows 134 -> 144, 20 rows 150 -> 156, 22 rows (0.69 in use) 162 -> 164, 28 rows 198 -> 193, 32 rows
+//   221 -> 199; with 32 heads 20 rows 91 -> 93, 22 rows 98.3 -> 97.9, 28 rows 117 -> 111.
 template <class W>
 uint32_t fa_score_tiles(const W & w, uint32_t D, uint32_t n_head, uint32_t T, const uint32_t * msum, uint32_t & lo) {
     lo = msum[8];
     if (D > 128u || (msum[3] & 1u) != 0u || w.cells * n_head * (D / 64u) < (10ull << 20) ||
         4u * w.cells * n_head >= (1ull << 31) || (uint64_t)T * n_head * D >= (1ull << 31))
         return 0u;
-    uint32_t n_map = 0;
+    uint32_t n_map = 0, n_blk = 0;                                // tiles of the longest row, of the 32 rows so far
+    uint64_t formed = 0;                                          // cells
     for (uint32_t t = 0; t < T; ++t) {
         const uint32_t * r = msum + 8u + 4u * t;
         if (r[0] != lo || r[1] <= r[0] || r[2] < r[3]) return 0u;
-        n_map = std::max(n_map, ((r[1] + 15u) / 16u - lo / 16u + 15u) / 16u);
+        n_blk = std::max(n_blk, ((r[1] + 15u) / 16u - lo / 16u + 15u) / 16u);
+        if (t % 32u != 31u && t + 1u < T) continue;
+        n_map = std::max(n_map, n_blk);
+        formed += 32u * 256u * (uint64_t)n_blk;
+        n_blk = 0;
     }
+    if (3u * w.cells < 2u * formed) return 0u;
     for (const FaItem & it : w.items)
         if (((it.u0 - lo / 16u) & 15u) != 0u) return 0u;
     return n_map;

@@ -60,13 +60,14 @@ static const char * check_layout(const FaWork & w, uint32_t T, uint32_t n_head, 
 }
 
 int main() {
-    size_t taken = 0, refused = 0, cut = 0;
+    size_t taken = 0, refused = 0, cut = 0, sparse = 0;
     for (uint32_t nkv = 1; nkv <= 64; ++nkv)
         for (uint32_t D : { 64u, 128u })
             for (uint32_t G : { 1u, 4u, 8u })
                 for (uint32_t lo : { 0u, 37u, 4096u })
                     for (uint32_t hist : { 300u, 1500u, 2048u, 2100u, 3600u, 9300u })
-                        for (uint32_t T : { 33u, 256u }) {
+                        for (uint32_t shape : { 9u, 20u, 23u, 33u, 62u, 256u, 1256u }) {
+                            const uint32_t T = shape % 1000u;     // 1256: one row in four long, the others of 40 cells
                             const uint32_t E = nkv * D, n_head = nkv * G;
                             if (n_head * D > 32768u || G * E > 32768u || E / 64u > 511u) continue;   // not shapes of the library
                             std::vector<uint32_t> msum(8u + 4u * T, 0u);
@@ -74,7 +75,7 @@ int main() {
                             msum[2] = lo + hist + T;
                             for (uint32_t t = 0; t < T; ++t) {
                                 msum[8u + 4u * t] = lo;
-                                msum[9u + 4u * t] = lo + hist + 1u + t;
+                                msum[9u + 4u * t] = lo + (shape > 1000u && t % 4u ? 40u : hist + 1u + t);
                             }
                             const uint32_t runs[1][2] = { { lo + hist, lo + hist + T } };
                             FaWork w;
@@ -86,18 +87,26 @@ int main() {
                                 const uint32_t n = (msum[9u + 4u * t] + 15u) / 16u - lo / 16u, ncg = ncg_of(E, D, n);
                                 aligned = aligned && (ncg % 16u == 0u || n <= ncg);
                             }
+                            uint64_t formed = 0;                  // cells of the tiles that a workgroup of 32 rows forms
+                            for (uint32_t b = 0; b < T; b += 32u) {
+                                uint32_t top = 0;
+                                for (uint32_t t = b; t < std::min(b + 32u, T); ++t) top = std::max(top, (msum[9u + 4u * t] + 15u) / 16u - lo / 16u);
+                                formed += 32u * 256u * (uint64_t)((top + 15u) / 16u);
+                            }
+                            const bool dense = 3u * w.cells >= 2u * formed;
                             const bool enough = w.cells * n_head * (D / 64u) >= (10ull << 20) && 4u * w.cells * n_head < (1ull << 31);
                             const char * bad = n_map ? check(w, T, n_head, n_map, first, msum.data()) : nullptr;
                             if (bad == nullptr) bad = check_layout(w, T, n_head, D, n_map);
-                            if (bad == nullptr && (n_map != 0u) != (aligned && enough)) bad = "the route's rule";
+                            if (bad == nullptr && (n_map != 0u) != (aligned && enough && dense)) bad = "the route's rule";
                             if (bad != nullptr) {
                                 printf("%s: %u of %u heads, D %u, %u rows behind %u cells from %u\n", bad, nkv, n_head, D, T, hist, lo);
                                 return 1;
                             }
                             taken += n_map != 0u;
                             refused += n_map == 0u;
-                            cut += enough && !aligned;
+                            cut += enough && dense && !aligned;
+                            sparse += enough && aligned && !dense;
                         }
-    printf("%zu work lists on the matrix cores, %zu not, %zu of them for their chunk cuts\n", taken, refused, cut);
-    return taken != 0u && cut != 0u ? 0 : 3;
+    printf("%zu work lists on the matrix cores, %zu not, %zu of them for their chunk cuts, %zu as too sparse\n", taken, refused, cut, sparse);
+    return taken != 0u && cut != 0u && sparse != 0u ? 0 : 3;
 }

@@ -92,7 +92,9 @@ def test_fa_causal_prefill_baseline_512(dev, oc):
 ], ids=["ragged", "lo37", "d64", "t9", "special"])
 def test_fa_rows_matrix_core_scores(dev, oc, T, lo, hist, n_head, n_head_kv, D, special):
     """Many rows with one run each from a common cell: enough scores (n_head x cells x D / 64 >= 10 x 2^20)
-    for the matrix-core score kernel. Row t sees cells [lo, hist + t], the rows' cells planned newest last."""
+    for the matrix-core score kernel. Row t sees cells [lo, hist + t], the rows' cells planned newest last. Where
+    less than two thirds of the scores that it would form are in use (all but d64), the one-row kernel runs:
+    test_fa_rows_matrix_core_scores_dense has the shapes that reach it."""
     n, E = hist + T, n_head_kv * D
     assert sum((hist + t + 16) // 16 * 16 - lo // 16 * 16 for t in range(T)) * n_head * (D // 64) >= 10 << 20
     kc, vc = _cache(oc, n, E, T + D)
@@ -116,6 +118,43 @@ def test_fa_rows_matrix_core_scores(dev, oc, T, lo, hist, n_head, n_head_kv, D, 
     out = dev.alloc(4 * T * n_head * D)
     dev.flash_attn(dev.upload(q), T, n_head * D, K_, V_, D, n_head, n_head_kv, scale, msum, out, n_head * D,
                    new_runs=[[hist, n]])
+    assert_bits_equal(out.read(np.float32, (T, n_head * D)), want, f"{T} rows behind {hist}")
+
+
+@pytest.mark.parametrize("T,lo,hist,n_head,n_head_kv,D,special", [
+    (30, 0, 2780, 64, 8, 128, None),      # one row block of 30 rows, 11 tiles less a part, two chunks a row
+    (62, 37, 1340, 64, 8, 128, None),     # the runs start inside a group; a ragged second row block
+    (25, 5, 6400, 64, 8, 128, None),      # several chunks a row, cut from the runs' first group on
+    (96, 0, 1920, 64, 1, 64, None),       # D 64, one KV head; the third row block begins a tile of its own
+    (30, 0, 2780, 64, 8, 128, "scales"),  # NaN / Inf / largest scales of K and V, zero and NaN queries
+], ids=["one_block", "lo37", "chunks", "d64", "special"])
+def test_fa_rows_matrix_core_scores_dense(dev, oc, T, lo, hist, n_head, n_head_kv, D, special):
+    """Rows that fill the tiles of the matrix-core score kernel to two thirds and more (the condition to run it)."""
+    n, E = lo + hist + T, n_head_kv * D
+    groups = (lo + hist + np.arange(T) + 16) // 16 - lo // 16
+    formed = sum(32 * 16 * 16 * ((int(groups[b:b + 32].max()) + 15) // 16) for b in range(0, T, 32))
+    assert 3 * 16 * int(groups.sum()) >= 2 * formed and 16 * int(groups.sum()) * n_head * (D // 64) >= 10 << 20
+    kc, vc = _cache(oc, n, E, T + D)
+    q = S.normal(T, T * n_head * D).reshape(T, n_head * D)
+    if special:
+        k, v = kc.reshape(n, E // 32, 34), vc.reshape(n, E // 32, 34)
+        for row, b, bits in ((5, 1, 0x7C00), (300, 9, 0xFC00), (901, 17, 0x7E00), (1500, 26, 0x7BFF)):
+            k[row, b, :2] = np.array([bits], np.uint16).view(np.uint8)
+            v[row + 1, b, :2] = np.array([bits], np.uint16).view(np.uint8)
+        v[:, 30, :2] = np.array([0x0001], np.uint16).view(np.uint8)       # the smallest scale: tiny weights
+        q[3, :128], q[7, 640] = 0.0, np.nan
+        q[11] *= np.float32(60.0)                                         # most weights underflow to zero
+    msum = np.zeros(8 + 4 * T, np.uint32)
+    msum[0], msum[1], msum[2] = 0x4D55534D, T, n
+    msum[8::4], msum[9::4] = lo, lo + hist + 1 + np.arange(T)
+    scale = np.float32(1.0 / math.sqrt(D))
+    want = oc.flash_attn(q, kc, vc, D, n_head, n_head_kv, scale, msum, None, [[lo + hist, n]])
+    K_, V_ = dev.kv(E, n), dev.kv(E, n)
+    K_.set_bytes(0, kc)
+    V_.set_bytes(1, vc)
+    out = dev.alloc(4 * T * n_head * D)
+    dev.flash_attn(dev.upload(q), T, n_head * D, K_, V_, D, n_head, n_head_kv, scale, msum, out, n_head * D,
+                   new_runs=[[lo + hist, n]])
     assert_bits_equal(out.read(np.float32, (T, n_head * D)), want, f"{T} rows behind {hist}")
 
 
