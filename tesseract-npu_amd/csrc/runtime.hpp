@@ -124,20 +124,24 @@ struct tsr_staging {
     }
 };
 
-// Pinned host slots for the work lists of unplanned FLASH_ATTN_EXT calls: the list is built in a slot and a
+// Pinned host slots for the long work lists of unplanned FLASH_ATTN_EXT calls: the list is built in a slot and a
 // kernel reads it from there into the scratch (tsr_launch_fetch). A slot is reused only after the kernel that
-// last read it has run (its event). Allocated at the first list (1 MB a context), given back with the context;
-// a list beyond a slot, or a context without the memory, takes a copy of pageable memory instead.
+// last read it has run (its event). Allocated at the first long list (1 MB a context), given back with the context;
+// a list beyond a slot, or a context without the memory, takes a copy of pageable memory instead, and so does a
+// list of at most kCopyBytes: the runtime stages such a copy itself and runs it as a kernel, without the event
+// (8 heads of D 64, a call in a queue of calls, copy -> slot: 700 bytes 19.5 -> 22.0 us, 13 KB 24.6 -> 28.0; one call
+// and its wait 27.3 -> 29.5 and 33.9 -> 36.4). Longer copies go to a copy engine, two hand-overs away from the
+// compute queue: 17.6 KB 34.8 -> 24.6 us, 66 KB 55 -> 46.
 struct tsr_lists {
     static constexpr uint32_t kSlots = 4;
-    static constexpr size_t kSlotBytes = (size_t)256 << 10;
+    static constexpr size_t kSlotBytes = (size_t)256 << 10, kCopyBytes = 16384;
     uint8_t * host = nullptr;
     hipEvent_t ev[kSlots] = {};
     bool used[kSlots] = {};
     bool tried = false;
     uint32_t next = 0;
     uint8_t * acquire(size_t bytes) {                             // nullptr: none for this list
-        if (bytes > kSlotBytes) return nullptr;
+        if (bytes > kSlotBytes || bytes <= kCopyBytes) return nullptr;
         if (!tried) {
             tried = true;
             bool ok = hipHostMalloc((void **)&host, kSlots * kSlotBytes, hipHostMallocCoherent) == hipSuccess;

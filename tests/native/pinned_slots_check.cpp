@@ -51,7 +51,8 @@ int tsr::hip_err(hipError_t e, const char *) { return e == hipSuccess ? 0 : TSR_
 int tsr_launch_fetch(void * dst, const void * host, size_t bytes, hipStream_t) { return enqueue(dst, host, bytes); }
 
 int main() {
-    uint8_t dst[64], src[64];
+    static uint8_t dst[64], src[64];
+    constexpr size_t kList = tsr_lists::kCopyBytes + 1u;
     for (int lists = 0; lists < 2; ++lists)
         for (int fail = -1; fail < 70; ++fail) {                  // which hipEventRecord fails (-1: none)
             for (int calls : { 1, 5, 70, 140 }) {
@@ -59,12 +60,13 @@ int main() {
                 n_events = 0;
                 tsr_lists l;
                 tsr_staging st;
+                if (l.acquire(tsr_lists::kCopyBytes) != nullptr || l.acquire(tsr_lists::kSlotBytes + 1u) != nullptr) return 3;
                 for (int i = 0; i < calls; ++i) {
                     if (lists) {
-                        uint8_t * slot = l.acquire(sizeof src);
+                        uint8_t * slot = l.acquire(kList);
                         if (slot == nullptr) return 2;
-                        memset(slot, i + 1, sizeof src);
-                        (void)l.send(dst, sizeof src, nullptr);
+                        memset(slot, i + 1, kList);
+                        (void)l.send(dst, kList, nullptr);
                     } else {
                         memset(src, i + 1, sizeof src);
                         (void)st.copy(dst, src, sizeof src, nullptr);

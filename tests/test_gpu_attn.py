@@ -186,10 +186,12 @@ def test_fa_rows_many_kv_heads(dev, oc, T, hist, n_head, n_head_kv, D):
     assert_bits_equal(out.read(np.float32, (T, n_head * D)), want, f"{T} rows of {n_head_kv} KV heads")
 
 
-@pytest.mark.parametrize("T,calls", [(40, 11), (7000, 2)], ids=["slots_reused", "list_beyond_a_slot"])
+@pytest.mark.parametrize("T,calls", [(40, 11), (372, 3), (373, 11), (7000, 2)],
+                         ids=["short_lists", "longest_copied", "slots_reused", "list_beyond_a_slot"])
 def test_fa_queued_work_lists(dev, oc, T, calls):
-    """Unplanned calls with work lists of their own queued behind each other without a wait: each sees its own
-    list, also when the pinned slots wrap (4) and when a list does not fit one (256 KB)."""
+    """Unplanned calls with work lists of their own (44 bytes a row) queued behind each other without a wait: each
+    sees its own list, as a copy of at most 16 KB, through the pinned slots when these wrap (4), and when a list does
+    not fit a slot (256 KB)."""
     n, nh, nkv, D = 300, 2, 1, 64
     kc, vc = _cache(oc, n, nkv * D, T)
     K_, V_ = dev.kv(nkv * D, n), dev.kv(nkv * D, n)
