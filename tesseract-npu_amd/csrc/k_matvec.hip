@@ -437,7 +437,7 @@ __global__ __launch_bounds__(1024) void k_mv_q4k(MvArgs a) {
 // an fp16 value, so every term is exact with plain IEEE operations.
 // ---------------------------------------------------------------------------------------------
 template <int P, bool ISUMS, int PREP, bool GLU>
-__global__ __launch_bounds__(1024) void k_mv_q80(MvArgs a) {
+__device__ __forceinline__ void mv_q80(const MvArgs & a) {
     extern __shared__ __align__(16) uint8_t lds[];
     const WGeom g = wgeom(a.N, a.K >> 5, a.rb, false);
     const uint32_t nb = g.nb, kx = g.q + (g.rem ? 1u : 0u);
@@ -546,6 +546,18 @@ __global__ __launch_bounds__(1024) void k_mv_q80(MvArgs a) {
     mv_tree_store<GLU>(a, s_p, s_t, nrow, row_lo, t, false, t64, add0);
 }
 
+// Without the norm two workgroups share a CU, also by their scalar registers: 80 at most (compiled freely they are
+// 81 to 84 with the rounding of a32_pack, and then the rounds of a few-row call run one workgroup at a time:
+// 4864x2048, 15 rows 30.2 -> 45.3 us). The norm's registers leave one workgroup in any case.
+template <int P, bool ISUMS, bool GLU>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_num_sgpr(80))) void k_mv_q80(MvArgs a) {
+    mv_q80<P, ISUMS, kPrepNone, GLU>(a);
+}
+template <int P, bool GLU>
+__global__ __launch_bounds__(1024) void k_mv_q80_norm(MvArgs a) {
+    mv_q80<P, false, kPrepNorm, GLU>(a);
+}
+
 }  // namespace tsr
 
 // ---- launchers ------------------------------------------------------------------------------------
@@ -595,24 +607,16 @@ static void launch_q4k_v(const tsr::MvArgs & a, dim3 grid, size_t lds, hipStream
         else launch_q4k<F, tsr::kPrepNone, false>(a, grid, lds, s);
     }
 }
-template <int P, int PREP, bool GLU>
-static void launch_q80(const tsr::MvArgs & a, dim3 grid, size_t lds, hipStream_t s) {
-    if constexpr (PREP == tsr::kPrepNone && !GLU) {
-        if (a.isums) {
-            hipLaunchKernelGGL((tsr::k_mv_q80<P, true, PREP, GLU>), grid, dim3(1024), lds, s, a);
-            return;
-        }
-    }
-    hipLaunchKernelGGL((tsr::k_mv_q80<P, false, PREP, GLU>), grid, dim3(1024), lds, s, a);
-}
 template <int P>
 static void launch_q80_v(const tsr::MvArgs & a, dim3 grid, size_t lds, hipStream_t s) {
+    const dim3 block(1024);
     if (a.prep == tsr::kPrepNorm) {
-        if (a.glu) launch_q80<P, tsr::kPrepNorm, true>(a, grid, lds, s);
-        else launch_q80<P, tsr::kPrepNorm, false>(a, grid, lds, s);
+        if (a.glu) hipLaunchKernelGGL((tsr::k_mv_q80_norm<P, true>), grid, block, lds, s, a);
+        else hipLaunchKernelGGL((tsr::k_mv_q80_norm<P, false>), grid, block, lds, s, a);
     } else {
-        if (a.glu) launch_q80<P, tsr::kPrepNone, true>(a, grid, lds, s);
-        else launch_q80<P, tsr::kPrepNone, false>(a, grid, lds, s);
+        if (a.isums) hipLaunchKernelGGL((tsr::k_mv_q80<P, true, false>), grid, block, lds, s, a);
+        else if (a.glu) hipLaunchKernelGGL((tsr::k_mv_q80<P, false, true>), grid, block, lds, s, a);
+        else hipLaunchKernelGGL((tsr::k_mv_q80<P, false, false>), grid, block, lds, s, a);
     }
 }
 
