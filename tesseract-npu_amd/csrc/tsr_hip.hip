@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "kernels.hpp"
+#include "mm_route.hpp"
 #include "runtime.hpp"
 #include "wlayout.hpp"
 
@@ -583,12 +584,11 @@ static int mul_mat_locked(tsr_hip_ctx * ctx, const tsr_hip_weight * w, const flo
         }
         return TSR_HIP_OK;
     }
-    // The matvec (one row; the integer sums; a workgroup per row and row block) or, for several rows, k_matrows.hip
-    // (the weights once per 15 rows; the fused norm form comes here at any T). As long as the matvec's
-    // workgroups run side by side, one a CU, it is the faster one: Q4_K 1024x2048, 4 rows 4.3 us against 4.9;
-    // beyond that it never is: 2048x2048, 3 rows 7.1 against 4.8, Q8_0 4096x4096, 2 rows 8.2 against 7.5.
+    // the matvec (one row; the integer sums) or, for several rows, the few-row kernels where they pay (the fused norm
+    // form comes here at any T)
     const uint32_t blocks = (w->N + w->rb - 1u) / w->rb;
-    const bool rows = isums == nullptr && (uint64_t)blocks * T > ctx->n_cu && T > 1u;
+    const bool rows = isums == nullptr && T > 1u &&
+                      tsr::few_rows_pay(w->fmt == TSR_HIP_FMT_Q4_K, w->K, w->rb, blocks, T, prep != nullptr, (uint32_t)ctx->n_cu);
     for (uint32_t t0 = 0; t0 < T; t0 += 65535u) {
         const uint32_t tt = std::min(T - t0, 65535u);
         a.x = x_dev + (size_t)t0 * x_stride;

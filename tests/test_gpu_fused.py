@@ -144,7 +144,8 @@ def test_mul_mat_glu(dev, oc, fmt, F, K, T, norm):
     (H.FMT_Q4_K, 20000, 2048, 15, "glu"),   # row chunks over one quantization
     (H.FMT_Q4_K, 5000, 1024, 31, "norm"),   # shares of 11, 11 and 9 tokens
     (H.FMT_Q4_K, 4130, 8192, 8, "norm"),
-    (H.FMT_Q8_0, 4100, 32, 2, "acc"),       # one block
+    (H.FMT_Q8_0, 4100, 32, 2, "acc"),       # one block (two rows: on the matvec)
+    (H.FMT_Q8_0, 4100, 32, 6, "acc"),       # one block
     (H.FMT_Q8_0, 4127, 1056, 4, "add"),     # odd rows; three blocks for one wave
     (H.FMT_Q8_0, 8222, 544, 7, "none"),
     (H.FMT_Q8_0, 20000, 1024, 9, "glu"),    # row chunks over one quantization
