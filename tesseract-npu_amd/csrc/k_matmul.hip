@@ -31,6 +31,7 @@
 // r = 0..15.
 #include "expk.hpp"
 #include "kernels.hpp"
+#include "mm_route.hpp"
 #include "qact.hpp"
 #include "wlayout.hpp"
 
@@ -252,31 +253,29 @@ __device__ __forceinline__ uint32_t q4k_sc(const uint4 mt, uint32_t j) {
     return __builtin_amdgcn_ubfe(j < 4u ? mt.y : mt.z, 8u * (j & 3u), 6);
 }
 // Work split. A workgroup of W = 4 waves (8: see the launcher) computes a tile of 32 weight rows x 32 tokens.
-// Wave j runs over the super-blocks of PG = 16 / W consecutive partials, which are consecutive slots of the weight layout, and folds
-// each finished partial into its subtree of the 16-partial tree, parking the left halves of the open
-// levels in LDS; the W subtrees meet in LDS at the end. (An empty partial is +0, and a sum that starts
-// at +0 is never -0, so folding one in changes nothing. With at most 8 or 4 super-blocks the higher
-// partials are empty, and PG shrinks so that every wave has work.) Eight waves with every load waited for
-// and all 16 partials in LDS, as this kernel had it, left a wave two super-blocks to set up and finish for.
+// Wave j runs over the super-blocks of its partials (mm_route.hpp: one or two pairs of neighbours, or two single
+// ones), whose sums are subtrees of the 16-partial tree: the first of a pair waits in LDS for the second, and the
+// waves' sums meet in LDS at the end. (An empty partial is +0, and a sum that starts at +0 is never -0, so adding one
+// changes nothing. The partials in use shrink with the row, so that every wave has work down to 3 super-blocks.)
 //
 // Loads. A register is requested again for the next super-block right behind its last use, so that a load
 // has a super-block's work (~3 waves on the SIMD) to arrive. Every load is made on every path and in one
 // order (the scheduling barriers): the counted waits then cover the loads they are for and no others, and
 // no register with a load in flight is copied.
 //
-// What bounds it (512 x 28672 x 4096 with GLU, counters): the VALU, ~84% busy: per tile and super-block 96
-// instructions for the terms (6 per output), ~150 to unpack and scale the weight quants, the rest set-up
-// and epilogue; the matrix cores 30%. Measured, before -> now: that shape 360 -> 250 us, 100 x 4096 x 4096
-// 16.6 -> 15.6, a Llama-3-8B layer over 300 tokens 537 -> 463. Splitting the partials over 2 waves or 1
-// instead of 4 gave 239 / 265 us there and 20 / 36 us at 100 tokens; 64 tokens a wave (unpacked weights used
-// twice) 328 us at the 2 waves a SIMD that its registers leave.
+// What bounds it: the VALU; per tile and super-block 96 instructions for the terms (6 per output), ~150 to unpack and
+// scale the weight quants, the rest set-up and epilogue. 512 x 28672 x 4096 with GLU, whole call: one workgroup of
+// eight waves a CU with every load waited for 326 us, four waves of four neighbouring partials each 252, with even
+// shares 237. There, with neighbours, two waves a tile took 239 us and one 265, but 100 x 4096 x 4096 20 and 36 us
+// instead of 15; 64 tokens a wave (unpacked weights used twice) 328 us at the 2 waves a SIMD that its registers leave.
 //
 // GLU: weight rows 2j and 2j + 1 are the gate and up rows of output j, in adjacent lanes: the even lane
 // forms y = SWIGLU(gate, up) of the even tokens, the odd lane of the odd ones.
 template <bool GLU, uint32_t W>
 __global__ __launch_bounds__(64 * W, W == 4u ? 3 : 2) void k_mm_q4k(MmArgs a) {
-    constexpr int kLev = W == 4u ? 2 : 1;                          // open tree levels of a wave
-    __shared__ float4 s_p[W][kLev][4][64];                         // wave, level: values r = 4 q + e of a lane
+    constexpr uint32_t V = 16u / W;                                // values of a lane that a wave finishes
+    typedef float vv_t __attribute__((ext_vector_type(V)));
+    __shared__ __align__(16) vv_t s_p[2][W][W][64];                // half, wave: values r = V q + e of a lane
     __shared__ int s_slow[W];
     const WGeom g = wgeom(a.N, a.K >> 8, a.rb, true);
     const uint32_t lane = __lane_id(), j = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -294,15 +293,16 @@ __global__ __launch_bounds__(64 * W, W == 4u ? 3 : 2) void k_mm_q4k(MmArgs a) {
     const uint64_t wend = B1 + 1u < g.nblk ? (uint64_t)(B1 + 1u) * g.bstride : wl_bytes(g);
     const __amdgpu_buffer_rsrc_t rw = brsrc(a.w + wbase, (uint32_t)(wend - wbase));
     const __amdgpu_buffer_rsrc_t rx = brsrc(a.qa, a.d_off + 4u * a.tp * g.nb);
-    const uint32_t np = g.nb > 8u ? 16u : (g.nb > 4u ? 8u : (g.nb > 2u ? 4u : g.nb));   // partials in use, a power of two
-    const uint32_t PG = max(np / W, 1u), w0 = PG * j;
-    const uint32_t sl0 = wl_slot(g, min(w0, 15u), 0u);
+    const MmSplit ms = mm_split(g.nb, W);
+    const uint32_t HP = ms.per, w0 = mm_partial(ms, j, 0u), w1 = mm_partial(ms, j, HP);   // first partial of each half
+    const bool both = ms.halves > 1u;
+    const uint32_t sl0 = wl_slot(g, w0, 0u);
     const uint32_t sR = 16u * R, sG = 32u * R * g.nb;
     uint32_t owq = (uint32_t)(wl_quant_off(g, B, R, h, sl0, rr) - wbase);   // piece 2 gg + h: + sG gg; + sR per slot
     uint32_t owm = (uint32_t)(wl_meta_off(g, B, R, sl0, rr) - wbase);
-    const uint32_t ox = 32u * t + 16u * h;                         // quants of sub-block jb: + 32 T jb
-    const uint32_t obs = a.s_off + 32u * t + 16u * h;              // sums (h_j, l_j), j = 4 h ..: + 32 T s
-    const uint32_t odx = h ? 0x80000000u : a.d_off + 4u * (t0 + c);   // token t0 + c's scale: + 4 tp s
+    uint32_t ox = 32u * t + 16u * h;                               // quants of sub-block jb: + 32 T jb
+    uint32_t obs = a.s_off + 32u * t + 16u * h;                    // sums (h_j, l_j), j = 4 h ..: + 32 T s
+    uint32_t odx = h ? 0x80000000u : a.d_off + 4u * (t0 + c);      // token t0 + c's scale: + 4 tp s
     const uint32_t m4 = 0x0F0F0F0Fu, T32 = 32u * a.T;
     typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
     // byte-wise q * f of a dword of quants q <= 15 and f <= 7 (no byte carries into the next: q f <= 105)
@@ -325,8 +325,13 @@ __global__ __launch_bounds__(64 * W, W == 4u ? 3 : 2) void k_mm_q4k(MmArgs a) {
     };
     bool slow = false;
     v16f p;
+    uint32_t t64 = 0;                                              // ahead of the loads that the epilogue does not wait for
+    if constexpr (GLU) t64 = a.ex.t64[lane];
+    __builtin_amdgcn_sched_barrier(0);
     uint32_t left = 0;                                             // super-blocks of this wave still to come
-    for (uint32_t pi = 0; pi < PG; ++pi) left += wl_count(g, w0 + pi);
+    for (uint32_t pi = 0; pi < HP; ++pi) left += wl_count(g, w0 + pi);
+    const uint32_t sJ = both ? sR * (wl_slot(g, w1, 0u) - sl0 - left + 1u) : 0u;   // from the last slot of half 0 to half 1
+    for (uint32_t pi = 0; pi < HP && both; ++pi) left += wl_count(g, w1 + pi);
     if (left > 0u) {
         load_t();
         __builtin_amdgcn_sched_barrier(0);
@@ -336,15 +341,18 @@ __global__ __launch_bounds__(64 * W, W == 4u ? 3 : 2) void k_mm_q4k(MmArgs a) {
         load_m(w0);
         __builtin_amdgcn_sched_barrier(0);
     }
-    for (uint32_t pi = 0; pi < PG; ++pi) {
-    const uint32_t pj = w0 + pi, cnt = wl_count(g, pj);
+    for (uint32_t pi = 0; pi < ms.halves * HP; ++pi) {
+    const uint32_t hf = pi < HP ? 0u : 1u, pj = mm_partial(ms, j, pi), cnt = wl_count(g, pj);
     p = (v16f){};
     for (uint32_t k = 0; k < cnt; ++k) {
         const uint32_t s = pj + 16u * k;
         --left;
-        // the next super-block (the last one again when there is none: a valid load that nothing uses)
-        const uint32_t sn = left == 0u ? s : (k + 1u < cnt ? s + 16u : pj + 1u);
-        if (left > 0u) { owq += sR; owm += sR; }
+        // the next super-block; behind the last one offsets past the windows' ends, whose loads touch no memory (the last
+        // one's again instead: 28672x4096, 128 rows 66 -> 72 us)
+        const bool jump = k + 1u == cnt && pi + 1u == HP;          // to half 1
+        const uint32_t sn = left == 0u ? s : (k + 1u < cnt ? s + 16u : (jump ? w1 : pj + 1u));
+        if (left > 0u) { owq += jump ? sJ : sR; owm += jump ? sJ : sR; }
+        else { owq = owm = ox = obs = odx = 0x80000000u; }
         const uint4 mc = mt;
         __builtin_amdgcn_sched_barrier(0);                         // (a load in flight shares no register with a live value)
         load_t();
@@ -384,8 +392,8 @@ __global__ __launch_bounds__(64 * W, W == 4u ? 3 : 2) void k_mm_q4k(MmArgs a) {
             const uint32_t ad = fb(dxl) & 0x7FFFFFFFu;             // the 32 tokens' scales, one a lane
             slow = slow || __ballot(ad != 0u && ad < 0x21800000u) != 0ull;   // wave-uniform, sticky
         }
-        v16f ms = {};
-        ms = __builtin_amdgcn_mfma_f32_32x32x16_f16(bs, mb, ms, 0, 0, 0);
+        v16f msum = {};
+        msum = __builtin_amdgcn_mfma_f32_32x32x16_f16(bs, mb, msum, 0, 0, 0);
         if (!slow) {
             // d Dx and dmin Dx as outer products on the matrix core (one IEEE product each; k = 1 is zero)
             v16f P1 = {}, P2 = {};
@@ -393,7 +401,7 @@ __global__ __launch_bounds__(64 * W, W == 4u ? 3 : 2) void k_mm_q4k(MmArgs a) {
             P2 = __builtin_amdgcn_mfma_f32_32x32x2f32(dxl, h ? 0.0f : dm, P2, 0, 0, 0);
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const float tt = P1[r] * (float)((ia[r] << 3) + ib[r]) - P2[r] * ms[r];
+                const float tt = P1[r] * (float)((ia[r] << 3) + ib[r]) - P2[r] * msum[r];
                 p[r] = p[r] + tt;
             }
         } else {
@@ -402,7 +410,7 @@ __global__ __launch_bounds__(64 * W, W == 4u ? 3 : 2) void k_mm_q4k(MmArgs a) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const float dx = xd[8 * (r >> 2) + (r & 3)];
-                const float tt = ssub(smul(smul(d, dx), i2f((ia[r] << 3) + ib[r])), smul(smul(dm, dx), ms[r]));
+                const float tt = ssub(smul(smul(d, dx), i2f((ia[r] << 3) + ib[r])), smul(smul(dm, dx), msum[r]));
                 p[r] = sadd(p[r], tt);
             }
         }
@@ -410,57 +418,54 @@ __global__ __launch_bounds__(64 * W, W == 4u ? 3 : 2) void k_mm_q4k(MmArgs a) {
         load_m(sn);
         __builtin_amdgcn_sched_barrier(0);
     }
-    // fold the partial into the tree (the wave's own lanes in LDS): bit lv of pi set: it is the right half
-    // of level lv, else the left half, parked. The last partial has every bit set and stays in p.
-    bool open = true;
+    // the second partial of a half meets the first one, parked in LDS (the wave's own lanes)
+    vv_t (*sp)[64] = s_p[hf][j];
+    if (pi + 1u == (hf + 1u) * HP && HP > 1u) {                    // wave-uniform
+        float u[16];
 #pragma unroll
-    for (int lv = 0; lv < kLev; ++lv) {
-        if (!open || (1u << lv) >= PG) continue;                   // wave-uniform
-        float4 (*sp)[64] = s_p[j][lv];
-        if ((pi >> lv) & 1u) {
+        for (uint32_t r = 0; r < 16u; ++r) u[r] = sp[r / V][lane][r % V];
+        if (__builtin_expect(!slow, 1)) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const float4 u = sp[q][lane];
-                if (!slow) {
-                    p[4 * q] = u.x + p[4 * q]; p[4 * q + 1] = u.y + p[4 * q + 1];
-                    p[4 * q + 2] = u.z + p[4 * q + 2]; p[4 * q + 3] = u.w + p[4 * q + 3];
-                } else {
-                    p[4 * q] = sadd(u.x, p[4 * q]); p[4 * q + 1] = sadd(u.y, p[4 * q + 1]);
-                    p[4 * q + 2] = sadd(u.z, p[4 * q + 2]); p[4 * q + 3] = sadd(u.w, p[4 * q + 3]);
-                }
-            }
+            for (uint32_t r = 0; r < 16u; ++r) p[r] = u[r] + p[r];
         } else {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) sp[q][lane] = make_float4(p[4 * q], p[4 * q + 1], p[4 * q + 2], p[4 * q + 3]);
-            open = false;
+            for (uint32_t r = 0; r < 16u; ++r) p[r] = sadd(u[r], p[r]);
         }
     }
-    }
 #pragma unroll
-    for (int q = 0; q < 4; ++q) s_p[j][0][q][lane] = make_float4(p[4 * q], p[4 * q + 1], p[4 * q + 2], p[4 * q + 3]);
+    for (uint32_t q = 0; q < W; ++q) {
+        vv_t v;
+#pragma unroll
+        for (uint32_t e = 0; e < V; ++e) v[e] = p[V * q + e];
+        sp[q][lane] = v;
+    }
+    }
     if (lane == 0u) s_slow[j] = slow ? 1 : 0;
-    uint32_t t64 = 0;
-    if constexpr (GLU) t64 = a.ex.t64[lane];
     lds_barrier();
 
     // wave j finishes V values of each lane, r = V j + e: weight row n0 + lane % 32, tokens t4 + e
-    constexpr uint32_t V = 16u / W;
     int any_slow = 0;
-    float u[W][V];
+    vv_t u[2u * W];
 #pragma unroll
-    for (uint32_t i = 0; i < W; ++i) {
-        any_slow |= s_slow[i];
-        const float * sp = (const float *)&s_p[i][0][V * j >> 2][lane] + (V * j & 3u);
-#pragma unroll
-        for (uint32_t e = 0; e < V; ++e) u[i][e] = sp[e];
+    for (uint32_t i = 0; i < 2u * W; ++i) {
+        if (i < W) any_slow |= s_slow[i];
+        u[i] = i < W || both ? s_p[i / W][i % W][j][lane] : (vv_t){};
     }
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(any_slow) == 0, 1)) {
 #pragma unroll
-    for (uint32_t m = W / 2u; m > 0u; m >>= 1)
+        for (uint32_t m = W; m > 0u; m >>= 1)
 #pragma unroll
-        for (uint32_t i = 0; i < m; ++i)
+            for (uint32_t i = 0; i < m; ++i)
 #pragma unroll
-            for (uint32_t e = 0; e < V; ++e)
-                u[i][e] = any_slow ? sadd(u[2u * i][e], u[2u * i + 1u][e]) : u[2u * i][e] + u[2u * i + 1u][e];
+                for (uint32_t e = 0; e < V; ++e) u[i][e] = u[2u * i][e] + u[2u * i + 1u][e];
+    } else {
+#pragma unroll
+        for (uint32_t m = W; m > 0u; m >>= 1)
+#pragma unroll
+            for (uint32_t i = 0; i < m; ++i)
+#pragma unroll
+                for (uint32_t e = 0; e < V; ++e) u[i][e] = sadd(u[2u * i][e], u[2u * i + 1u][e]);
+    }
     float v[V];
 #pragma unroll
     for (uint32_t e = 0; e < V; ++e) v[e] = canon(u[0][e]);
@@ -507,15 +512,13 @@ int tsr_launch_mm_q4_k(const tsr::MmArgs & a, uint32_t n_cu, hipStream_t s) {
     tsr::MmArgs m = a;
     m.grouped = (gx & 7u) == 0u && (uint64_t)a.N * (a.K / 256u) * 144u > (48ull << 20) ? 1u : 0u;   // measured
     const dim3 grid = m.grouped ? dim3(8u * gy, gx / 8u) : dim3(gx, gy);
-    // Eight waves a tile while the tiles leave the chip short of waves (one tile a CU; with long rows, two): the
-    // chain of a wave's super-blocks is then the time. With more tiles the eight-wave form's one workgroup a CU
-    // loses to three of four waves. Four -> eight waves, us: 2048x14336, 33 rows 22.8 -> 18.2, 128 rows (256 tiles)
-    // 26.0 -> 21.5, 256 rows (512) 37.1 -> 35.1, 512 rows (1024) 59.7 -> 62.8; 4096x4096, 64 rows 11.8 -> 11.0,
-    // 100 rows (512 tiles) 15.1 -> 16.2; 4096x2048, 64 rows 8.9 -> 8.3; rows of 4 super-blocks, which eight waves
-    // cannot share, 700x1024, 50 rows 6.8 -> 7.3.
+    // Eight waves a tile while there is at most one tile a CU: the chain of a wave's super-blocks is then the time.
+    // With more, three workgroups of four waves a CU beat one of eight. Four -> eight waves, whole calls, us:
+    // 2048x14336, 64 rows (128 tiles) 22.3 -> 18.9, 128 rows (256) 25.2 -> 22.4, 256 rows (512) 38.0 -> 40.5;
+    // 4096x4096, 64 rows (256) 11.5 -> 10.8, 128 rows (512) 15.7 -> 18.2; 2048x5632, 160 rows (320) 18.3 -> 20.5; rows
+    // of 4 super-blocks, 512x1024, 512 rows (256) 7.7 -> 7.7, 4864x1024, 64 rows (304) 8.1 -> 9.6.
     const uint64_t tiles = (uint64_t)gx * gy;
-    const uint32_t nb = a.K >> 8;
-    const bool w8 = nb > 4u && (tiles <= n_cu || (tiles <= 2u * n_cu && nb >= 48u));
+    const bool w8 = tiles <= n_cu;
     if (w8) {
         if (a.glu) hipLaunchKernelGGL((tsr::k_mm_q4k<true, 8u>), grid, dim3(512), 0, s, m);
         else hipLaunchKernelGGL((tsr::k_mm_q4k<false, 8u>), grid, dim3(512), 0, s, m);

@@ -1,5 +1,5 @@
-// mm_route.hpp -- which kernels a MUL_MAT of several token rows runs on. Plain C++ without the HIP runtime, so
-// that it is checked on the CPU.
+// mm_route.hpp -- which kernels a MUL_MAT of several token rows runs on, and which partials a wave of the Q4_K
+// prefill kernel forms. Plain C++ without the HIP runtime, so that it is checked on the CPU.
 #pragma once
 
 #include <stdint.h>
@@ -42,6 +42,26 @@ inline bool few_rows_pay(bool q4k, uint32_t K, uint32_t rb, uint32_t blocks, uin
     }
     if (norm && rows > 8u && K > (q4k ? 7168u : 6144u)) s = 4u;
     return rounds((uint64_t)blocks * T) > s * rounds((uint64_t)blocks * shares);
+}
+
+// k_mm_q4k: the partials of wave j of W (4 or 8) for rows of nb super-blocks. The first nb mod 16 partials have one
+// super-block more than the others. A wave takes `per` neighbours from partials 0 .. 7 and the same ones of 8 .. 15,
+// subtrees of the 16-partial tree, or (halves 1) neighbours only.
+// Four waves, one a SIMD: two and two; four neighbours gave the first wave up to twice the others' work (2048x5632,
+// 160 rows 20.8 -> 18.4 us). Eight waves, j and j + 4 on one SIMD: one and one where that leaves the fullest SIMD a
+// super-block less (GLU 896x4864, 64 rows 11.6 -> 10.6 us), else two neighbours, whose sum goes through LDS once
+// (2048x5632, 64 rows 12.2 -> 11.4).
+struct MmSplit {
+    uint32_t halves, per;                                         // 2: both halves; partials in each
+};
+constexpr MmSplit mm_split(uint32_t nb, uint32_t W) {
+    const uint32_t np = nb > 4u ? 8u : (nb > 2u ? 4u : nb), rem = nb & 15u;   // partials in use in a half, a power of two
+    if (W == 8u && nb > 8u && !((rem >= 2u && rem <= 4u) || (rem >= 10u && rem <= 12u))) return { 1u, 2u };
+    return { nb > 8u ? 2u : 1u, np > W ? np / W : 1u };
+}
+// The wave's partial pi < halves * per, in the order it forms them.
+constexpr uint32_t mm_partial(const MmSplit & m, uint32_t j, uint32_t pi) {
+    return m.per * j + pi + (pi < m.per ? 0u : 8u - m.per);
 }
 
 }  // namespace tsr

@@ -212,12 +212,15 @@ def test_mm_q4_k_partial_counts(dev, oc, nsb):
 
 
 @pytest.mark.parametrize("N,nsb,T,glu", [
-    (8230, 9, 35, False),     # four waves: more tiles (516) than two a CU
+    (8230, 9, 35, False),     # four waves: 516 tiles
     (8230, 17, 35, True),
     (8230, 49, 35, False),
-    (8228, 49, 20, False),    # eight waves: 258 tiles of long rows
-    (8228, 16, 20, True),     # the same tiles of shorter rows: four
-    (1030, 23, 35, True),     # eight waves: one tile a CU
+    (8228, 49, 20, False),    # four waves: 258 tiles
+    (8228, 16, 20, True),
+    (1030, 23, 35, True),     # eight waves: 66 tiles, two neighbouring partials a wave
+    (1030, 12, 35, True),     # one partial of each half a wave
+    (1030, 20, 35, False),
+    (1030, 4, 35, False),     # fewer super-blocks than waves
 ], ids=lambda v: str(v))
 def test_mm_q4_k_wave_counts(dev, oc, N, nsb, T, glu):
     """The four- and eight-wave forms on both sides of the launcher's rule (256 CUs), with a token row whose
