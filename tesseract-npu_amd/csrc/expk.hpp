@@ -63,8 +63,8 @@ __device__ __forceinline__ float expk_diff(float s, float m, float scale, const 
 // integers, and with the f64 rounding mode set to truncation (f64_round_to_zero) fma(a, b, 2^52) holds
 // floor(a b) exactly in its low word. A step is a full-rate fma and add where the 32-bit form takes quarter-
 // rate integer products (~33 issue slots a value instead of ~60). v is cut off at -180, whose result is +0 as
-// that of everything below. Equal to the restatement of the reference on all 2^31 negative floats (a CPU
-// run in the truncating mode). td: t64[j] 2^-32 as f64, in LDS.
+// that of everything below. Equal to the oracle's EXPK on all 2^31 negative floats (tests/test_rounding.py, on the
+// CPU in the truncating mode). td: t64[j] 2^-32 as f64, in LDS.
 // The wave's f64 (and f16) operations truncate from here on (MODE.FP_ROUND[3:2] = toward zero); f32 keeps
 // rounding to nearest even. In asm, because the compiler takes a mode set by its builtin back in front of
 // the next f64 operation. x: a value on which every f64 operation meant depends (the only order that the

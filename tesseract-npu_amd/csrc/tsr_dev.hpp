@@ -107,7 +107,7 @@ __device__ __forceinline__ int32_t cvt_i32_sat(float x) {
 }
 __device__ __forceinline__ int32_t clamp8(int32_t v) { return min(max(v, -128), 127); }
 // Half away from zero: truncation of x + copysign(1/2 - 2^-25, x). The f32 sum reaches the next integer exactly
-// from fraction 1/2 on (checked against truncation and comparison for every f32 bit pattern).
+// from fraction 1/2 on (tests/test_rounding.py: every f32 bit pattern).
 __device__ __forceinline__ int32_t round_away(float x) { return cvt_i32_sat(x + __builtin_copysignf(0x1.fffffep-2f, x)); }
 __device__ __forceinline__ int32_t round_away8(float x) {
     return clamp8(round_away(x));                             // NaN -> 0, +-Inf -> 127 / -128
