@@ -53,7 +53,7 @@ namespace tsr {
 // The digits go to LDS as [block][head][digit][group][16 cells].
 // Phase B (matrix core): A[h][v] = sum_cells W[h][cell] q[cell][v] = sum_k 256^k sum_cells d_k q is
 // v_mfma_i32_16x16x64_i8 with rows (head, digit), columns 16 values and K the 64 cells; lane l then
-// holds the four digit sums of head l / 16 and value l % 16 and forms A exactly in f64.
+// holds the four digit sums of head l / 16 and value l % 16 and forms RNE24(A) (digits_rne24).
 // Every global load of the first batch is issued before the EXP work, so that a block waits for
 // memory once.
 // ---------------------------------------------------------------------------------------------
@@ -518,7 +518,8 @@ __global__ __launch_bounds__(256) void k_fa_qk(FaArgs a, FaPlan p) {
 // cell of 16 rows, so 32 lanes store 32 consecutive scores of a row. While every scale of the wave is finite
 // no score is Inf or NaN: the canonicalization and the NaN rule of the maximum are left to waves that met
 // one (sticky). The rows' store offsets are read from LDS where they are needed: with them in registers the
-// kernel spilled, and a reload waits for the stores in front of it (the memory counter retires in order).
+// kernel spilled them too, and a reload waits for the stores in front of it (the memory counter retires in order).
+// (D 128, at its 168 registers for three waves a SIMD: three of the 16 maxima pass through scratch once.)
 //
 // The one-row kernel below reads each K row per query row and spends ~130 VALU operations a score; this one
 // ~20.

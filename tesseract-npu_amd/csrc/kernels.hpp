@@ -77,7 +77,7 @@ struct MmArgs {
     uint32_t N, K, T;
     uint32_t acc;
     uint32_t rb;
-    // Q4_K (k_qact_mm4's A256 form): sub-block sums int32 [K/32][T] at qa + s_off, the super-block
+    // Q4_K (k_qact_mm4's A256 form): sub-block sums [K/256][T][8] at qa + s_off (64 h + l as f16 pairs (h, l)), the super-block
     // scales f32 [K/256][tp] at qa + d_off (tp: T rounded up to 32, padding tokens d = 0)
     uint32_t s_off, tp;
     uint32_t glu;            // Q4_K: rows 2j, 2j + 1 are gate / up of output j: y[j] = SWIGLU(gate, up)

@@ -17,9 +17,7 @@ __device__ __forceinline__ uint32_t mag_bits(float v) { return fb(daz(v)) & 0x7F
 
 __device__ __forceinline__ uint32_t umax_u(uint32_t a, uint32_t b) { return a > b ? a : b; }
 
-// One A32 block held by the 8 lanes of an aligned group: returns this lane's 4 quants packed
-// little-endian and the block's D in *D (every lane of the group).
-// Four quants of finite values with |x id| <= 127 (1 + 2^-22): no saturation. (With round_away as it is, 6 instead
+// Four quants, packed little-endian, of finite values with |x id| <= 127 (1 + 2^-22): no saturation. (With round_away as it is, 6 instead
 // of 11 instructions a value: the 4864x896 Q8_0 matvec, four launches 35.5 -> 33.8 us.)
 __device__ __forceinline__ uint32_t a32_pack(const float * xs, float id) {
     const uint32_t lo = __builtin_amdgcn_perm((uint32_t)round_away(xs[1] * id), (uint32_t)round_away(xs[0] * id), 0x0C0C0400u);
@@ -27,6 +25,8 @@ __device__ __forceinline__ uint32_t a32_pack(const float * xs, float id) {
     return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
 }
 
+// One A32 block held by the 8 lanes of an aligned group (qact_a32_lane): this lane's 4 quants packed little-endian
+// and the block's D in *D (every lane of the group).
 // The common case of qact_a32_lane: a wave whose values are all finite and whose blocks have amax = 0
 // or amax >= 2^-60. DAZ then acts on the maximum only (a subnormal maximum means a block of zeros after
 // DAZ), d = amax / 127 and RC(d) are plain IEEE operations on normal numbers, the plain product
