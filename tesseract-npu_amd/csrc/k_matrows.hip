@@ -14,7 +14,7 @@
 // about one tile a workgroup; then ~140 VALU instructions per tile and Q4_K super-block (2304 bytes), and the
 // quantization of every row in every workgroup (A32 ~8, A256 ~6, the norm ~7 instructions a value).
 // Against the matvec run once per row (the same box, us):
-//   Q4_K norm 6144x4096, 8 rows 40.7 -> 13.9; 4096x14336, 15 rows 93 -> 26; GLU norm 28672x4096, 8 rows 86 -> 28
+//   Q4_K norm 6144x4096, 8 rows 40.7 -> 13.3; 4096x14336, 15 rows 93 -> 26; GLU norm 28672x4096, 8 rows 86 -> 28
 //   Q8_0 4864x896, 8 rows 14.3 -> 6.1; 14336x4096, 8 rows 84 -> 15; 4096x14336, 15 rows 176 -> 34
 // Registers decide it: with 128 a wave, weights requested ahead of the quantization, or addresses kept over
 // the phases, spilled 20 to 60 of them and cost 5 to 20 us (mr_again; the rare paths in small steps).
