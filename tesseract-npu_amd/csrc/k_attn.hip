@@ -39,8 +39,7 @@ namespace tsr {
 
 // ---------------------------------------------------------------------------------------------
 // P.V: block (item * 4 + channel c, KV head g, group hg of 4 query heads x value part vh of VS); one
-// wave per segment of the channel (4 of its groups = 64 cells), looping if there are more segments
-// than waves. Each segment's results go to LDS; the f32 segment chain then runs in segment order.
+// wave per segment of the channel (4 of its groups = 64 cells). Each segment's results go to LDS; the f32 segment chain then runs in segment order.
 // A block covers D / VS values of its heads (VS > 1 when the grid would not fill the chip: the
 // value-independent EXP and LSUM work is then repeated per part, the value work is split).
 //
@@ -57,7 +56,7 @@ namespace tsr {
 // Every global load of the first batch is issued before the EXP work, so that a block waits for
 // memory once.
 // ---------------------------------------------------------------------------------------------
-constexpr uint32_t kPvWaves = 8;                                  // NCG <= 128 -> <= 8 segments per channel
+constexpr uint32_t kPvWaves = kMaxSegments;                       // one a segment
 
 // The P.V work of one block (chunk item, channel c, KV head g, head group hg, value part vh), shared by
 // k_fa_pv (the item's scores in global memory). Lane = (head row hr, group kk of the segment, cell quad);
@@ -151,13 +150,13 @@ struct PvBlock {
     }
 
     // One segment (L holds its loads): EXP, LSUM, the block-float weights, their digits and the
-    // matrix-core digit sums; the segment's results go to s_c [slot][4 heads][DV] and s_l [slot][4 heads].
+    // matrix-core digit sums; the segment's results go to s_c [seg][4 heads][DV] and s_l [seg][4 heads].
     // The common case of a batch (wave-uniform: every p and value scale finite, every head row's largest
     // weight 0 or in [2^-102, 2^106)) needs no flag and no flush: with the segment exponent E_S >= -102 a
     // subnormal weight rounds to W = 0 as the flushed one does, and with |A| in [1, 2^45) the scaled result
     // is a normal number for E_S in -102 .. 105. The general form runs otherwise.
     // Returns whether every batch was the common case.
-    __device__ __forceinline__ bool segment(uint32_t seg, uint32_t slot, Loads & L, float m, const ExpkNeg & en,
+    __device__ __forceinline__ bool segment(uint32_t seg, Loads & L, float m, const ExpkNeg & en,
                                             const double * s_td, float * s_c, float * s_l, uint8_t * dg) const {
         bool common = true;
         // ---- phase A: lane = (head row, 4 cells) ----------------------------------------------
@@ -183,7 +182,7 @@ struct PvBlock {
             for (int i = 0; i < 4; ++i) lsum += bf_int_n(pm >= 0x7F800000u ? 0.0f : pz[i], pe - 127);
             lsum = row16_isum(lsum);
             if ((lane & 15u) == 0u)
-                s_l[slot * 4u + hr] = pe == 255 ? bf(kNaN) : (pe == 0 ? 0.0f : bf_scale((float)lsum, pe - 150));
+                s_l[seg * 4u + hr] = pe == 255 ? bf(kNaN) : (pe == 0 ? 0.0f : bf_scale((float)lsum, pe - 150));
         }
 
 #pragma unroll
@@ -215,7 +214,7 @@ struct PvBlock {
                         const v4i_fa Bop = { bq.x, bq.y, bq.z, bq.w };
                         v4i_fa acc = { 0, 0, 0, 0 };
                         acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop, Bop, acc, 0, 0, 0);
-                        s_c[(slot * 4u + hr) * DV + 32u * (bt * BB + e) + 16u * (uint32_t)half + (lane & 15u)] =
+                        s_c[(seg * 4u + hr) * DV + 32u * (bt * BB + e) + 16u * (uint32_t)half + (lane & 15u)] =
                             __builtin_ldexpf(digits_rne24(acc), ef - 23);
                     }
                 }
@@ -269,7 +268,7 @@ struct PvBlock {
                     v4i_fa acc = { 0, 0, 0, 0 };
                     acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop, Bop, acc, 0, 0, 0);
                     const float cval = bad ? bf(kNaN) : (any[e >> 1] ? bf_scale(digits_rne24(acc), es[e >> 1] - 23) : 0.0f);
-                    s_c[(slot * 4u + hr) * DV + 32u * (bt * BB + e) + 16u * (uint32_t)half + (lane & 15u)] = cval;
+                    s_c[(seg * 4u + hr) * DV + 32u * (bt * BB + e) + 16u * (uint32_t)half + (lane & 15u)] = cval;
                 }
             }
         }
@@ -684,8 +683,8 @@ __global__ __launch_bounds__(64 * kPvWaves) void k_fa_pv(FaArgs a, FaPlan p) {
     using PB = PvBlock<D, VS>;
     constexpr uint32_t DV = PB::DV, BB = PB::BB;
     const uint32_t G = a.G, nh = a.n_head;
-    // the launch has one wave per segment of its longest channel (nw <= kPvWaves), so the segment
-    // results need nw slots: the LDS is sized by the launch
+    // the launch has one wave per segment of its longest channel (fa_segments), so the segment results need nw slots:
+    // the LDS is sized by the launch
     const uint32_t nw = blockDim.x >> 6;
     double * s_td = (double *)lds;                                // EXPK table
     float * s_c = (float *)(lds + 512);                           // [seg][4 heads][DV]
@@ -712,10 +711,10 @@ __global__ __launch_bounds__(64 * kPvWaves) void k_fa_pv(FaArgs a, FaPlan p) {
     float m = maxt_unkey(row16_umax(max(mkey, maxt_key_f(bf(kMFloor)))));
     f64_round_to_zero(m);
     bool common = true;
-    for (uint32_t seg = wave; seg < pb.nseg; seg += nw) {
-        if (seg != wave) pb.loads(seg, pb.vb0, L, true);
-        common = pb.segment(seg, seg, L, m, en, s_td, s_c, s_l, dg) && common;
-    }
+    // No loop (nseg <= nw): the loads of a second segment kept 24 to 36 more registers alive, 84 .. 100 instead of 60 .. 64,
+    // which left five waves a SIMD instead of eight. us, with the loop -> without: 512 rows behind 1536 cells, 32 / 8
+    // heads of D 128 177 -> 160; 1994 rows behind 130 882 -> 602; 1870 rows behind 246, 24 / 24 heads of D 64 1694 -> 1081.
+    if (wave < pb.nseg) common = pb.segment(wave, L, m, en, s_td, s_c, s_l, dg);
     pb.chains(item, hg, s_c, s_l, __syncthreads_and(common) != 0);
 }
 
@@ -892,7 +891,8 @@ static int launch_fa(const tsr::FaArgs & a, const tsr::FaPlan & p, uint32_t T, u
     } else {
         maxn = a.max_groups;
     }
-    const uint32_t nwv = std::max(1u, std::min(tsr::kPvWaves, ((maxn + 3u) / 4u + 3u) / 4u));
+    const uint32_t nwv = tsr::fa_segments(maxn);
+    if (nwv > tsr::kPvWaves) return -2;
     const uint64_t blocks = 4ull * p.n_items * a.n_head_kv * ((a.G + 3u) / 4u);
     uint32_t vs = 1;
     while (vs < 4u && a.D / (2u * vs) >= 64u && blocks * vs < 2ull * n_cu) vs *= 2u;

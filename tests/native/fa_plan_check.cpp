@@ -59,6 +59,19 @@ static const char * check_layout(const FaWork & w, uint32_t T, uint32_t n_head, 
     return apart(scores) && apart(rest) ? nullptr : "overlapping scratch";
 }
 
+// k_fa_pv has one wave per segment of the longest item: every channel of every item has to fit.
+static const char * check_segments(const FaWork & w) {
+    const uint32_t nw = fa_segments(w.max_groups);
+    if (nw > kMaxSegments) return "more segments than waves of a workgroup";
+    for (const FaItem & it : w.items)
+        for (uint32_t c = 0; c < kC; ++c) {                       // as PvBlock counts them
+            const uint32_t first = it.u0 + ((c + 4u - (it.u0 & 3u)) & 3u), end = it.u0 + it.n;
+            const uint32_t nu = first < end ? (end - 1u - first) / 4u + 1u : 0u;
+            if ((nu + 3u) / 4u > nw) return "a segment without a wave";
+        }
+    return nullptr;
+}
+
 int main() {
     size_t taken = 0, refused = 0, cut = 0, sparse = 0;
     for (uint32_t nkv = 1; nkv <= 64; ++nkv)
@@ -97,6 +110,7 @@ int main() {
                             const bool enough = w.cells * n_head * (D / 64u) >= (10ull << 20) && 4u * w.cells * n_head < (1ull << 31);
                             const char * bad = n_map ? check(w, T, n_head, n_map, first, msum.data()) : nullptr;
                             if (bad == nullptr) bad = check_layout(w, T, n_head, D, n_map);
+                            if (bad == nullptr) bad = check_segments(w);
                             if (bad == nullptr && (n_map != 0u) != (aligned && enough && dense)) bad = "the route's rule";
                             if (bad != nullptr) {
                                 printf("%s: %u of %u heads, D %u, %u rows behind %u cells from %u\n", bad, nkv, n_head, D, T, hist, lo);

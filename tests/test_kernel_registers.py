@@ -35,3 +35,11 @@ def test_q80_matvec_two_workgroups_a_cu(registers):
     k = {n: r for n, r in registers.items() if re.search(r"k_mv_q80ILi[12]E", n)}
     assert len(k) == 6
     assert all(s <= 80 and v <= 64 for s, v in k.values()), k
+
+
+def test_attention_pv_eight_waves_a_simd(registers):
+    """The P.V kernel of FLASH_ATTN_EXT: at most 64 vector registers, so that its workgroups of up to eight waves fill
+    the SIMDs."""
+    k = {n: r for n, r in registers.items() if re.search(r"k_fa_pvILi\d+E", n)}
+    assert len(k) == 18
+    assert all(v <= 64 for _, v in k.values()), k
