@@ -37,6 +37,13 @@ def test_q80_matvec_two_workgroups_a_cu(registers):
     assert all(s <= 80 and v <= 64 for s, v in k.values()), k
 
 
+def test_rope_kv_four_workgroups_a_cu(registers):
+    """ROPE + SET_ROWS_KV: four workgroups of eight waves on a CU (64 vector, 80 scalar registers)."""
+    k = {n: r for n, r in registers.items() if "k_rope_kv" in n}
+    assert len(k) == 1
+    assert all(s <= 80 and v <= 64 for s, v in k.values()), k
+
+
 def test_attention_pv_eight_waves_a_simd(registers):
     """The P.V kernel of FLASH_ATTN_EXT: at most 64 vector registers, so that its workgroups of up to eight waves fill
     the SIMDs."""
