@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark of the quantized-inference hot path on one MI355X.
 
-Headline workload (BASELINE.json configs[4], the configuration the metric is quoted on): greedy
+Headline workload (the configuration the metric is quoted on): greedy
 decode of a random-init Llama-3-8B-architecture model at batch 1 -- 32 layers, hidden 4096, FFN
 14336 SwiGLU, 32 q / 8 KV heads, head_dim 128, vocab 128256, every weight matrix (output head
 included) Q4_K from seeded N(0, 0.02), q8_0 KV caches prefilled through the model with 4096 seeded
@@ -17,7 +17,7 @@ takes the largest share of a token (its launch duration measured live with HIP e
 stream over the model's own layers), HBM traffic of that kernel from two rocprofv3 --pmc passes, and
 the CPU baseline: this repository's oracle (the reference's numerics restated in C) decoding the same
 model on the host cores -- whose first-token logits are also compared bit for bit with the GPU's.
-The other BASELINE configs (Q4_K FFN pair, Q8_0 matvec, flash-decode at 8192 cells, prefill) are
+The other workloads (Q4_K FFN pair, Q8_0 matvec, flash-decode at 8192 cells, prefill) are
 reported under "also".
 """
 from __future__ import annotations
@@ -157,7 +157,7 @@ def token_bytes(cfg, n_kv_read: int) -> int:
 
 
 def e2e_decode(dev, ev, steps: int, warmup: int, eager: bool = False) -> dict:
-    """BASELINE configs[4]: Llama-3-8B-architecture Q4_K decode with CTX cells of context.
+    """Llama-3-8B-architecture Q4_K decode with CTX cells of context.
 
     Cells 0 .. CTX-1 of every layer's caches are filled by the prefill of CTX random token ids in
     ubatches of UBATCH (untimed; its rate is reported); token 0, the prompt's greedy token, is decoded
@@ -344,7 +344,7 @@ def cpu_decode(e2e: dict, max_seconds: float = 40.0, max_tokens: int = 5) -> dic
 
 
 def cpu_configs(threads: int, runs: int = 5) -> dict:
-    """The oracle (the reference's numerics restated in C, oracle/oc_*.c) on BASELINE configs[0]-[3]'s
+    """The oracle (the reference's numerics restated in C, oracle/oc_*.c) on the single-op workloads'
     workloads, drawn from the same seeds as the GPU legs under "also", on the host cores: each at one
     thread and at `threads` threads, the median of `runs` timed runs after one untimed run. MUL_MAT is
     threaded over output rows (like the reference's mvm_rows pool, sw/sim/tsr_sim.c:1608-1647); the
@@ -377,14 +377,14 @@ def cpu_configs(threads: int, runs: int = 5) -> dict:
         return r
 
     out = {"runs": runs, "statistic": "median", "kind": "port", "threads_all": threads, "host": host_info()}
-    # configs[0]: Q8_0 matvec 4864 x 896 (the GPU leg's seeds)
+    # Q8_0 matvec 4864 x 896 (the GPU leg's seeds)
     N, K = 4864, 896
     w = S.quant_rows(0, S.seed_of("cfg1", "w"), N, K)
     x = S.normal(S.seed_of("cfg1", "x"), K)
     nb = N * (K // 32) * 34 + 4 * K + 4 * N
     out["q8_0_matvec_4864x896"] = both(lambda th: oc.mul_mat(0, w, K, x, threads=th),
                                        lambda s: {"us_per_call": round(s * 1e6, 1), "GB/s": round(nb / s / 1e9, 3)})
-    # configs[1]: Q4_K up 14336 x 4096 then down 4096 x 14336
+    # Q4_K up 14336 x 4096 then down 4096 x 14336
     up = S.quant_rows(1, S.seed_of("cfg2", "w_up"), 14336, 4096)
     dn = S.quant_rows(1, S.seed_of("cfg2", "w_down"), 4096, 14336)
     xu = S.normal(S.seed_of("cfg2", "x"), 4096)
@@ -396,7 +396,7 @@ def cpu_configs(threads: int, runs: int = 5) -> dict:
     out["ffn_pair_q4k_14336x4096_4096x14336"] = both(pair, lambda s: {"us_per_step": round(s * 1e6, 1),
                                                                       "GB/s": round(nb / s / 1e9, 3)})
     del up, dn
-    # configs[2]: FLASH_ATTN_EXT decode, 8192 cells, 32 q / 8 KV heads, D 128
+    # FLASH_ATTN_EXT decode, 8192 cells, 32 q / 8 KV heads, D 128
     n_kv, E = 8192, 1024
     kc = np.zeros((n_kv, E // 32 * 34), np.uint8)
     vc = np.zeros_like(kc)
@@ -411,7 +411,7 @@ def cpu_configs(threads: int, runs: int = 5) -> dict:
                                                             "GB/s": round(nb / s / 1e9, 3)},
                                               "note": "one sequential call (the plan spans all KV heads)"}
     del kc, vc
-    # configs[3]: prefill MUL_MATs (a 32-row sample of the 512 token rows) and the causal FA over 512 tokens
+    # prefill MUL_MATs (a 32-row sample of the 512 token rows) and the causal FA over 512 tokens
     T, K, Ts = 512, 4096, 32
     xs = S.normal(S.seed_of("cfg4", "x"), T * K).reshape(T, K)[:: T // Ts][:Ts]
     for name, N in (("prefill_q8_0_512x4096x4096", 4096), ("prefill_q8_0_512x14336x4096", 14336)):
@@ -530,9 +530,9 @@ def adapter_decode(ev, e2e, caches, steps: int) -> dict:
 
 
 def extra_workloads(dev, ev, stream, n: int, eager: bool = False) -> dict:
-    """The other single-GPU BASELINE configs, each timed over rotating device copies (> 2x MALL):
-    configs[1] the Q4_K FFN up/down pair, configs[0] Q8_0 matvec 4864x896, configs[2] q8-KV
-    flash-decode (32 q / 8 KV heads, D 128, n_kv 8192, batch 1), configs[3] the prefill matmuls and
+    """The single-op workloads, each timed over rotating device copies (> 2x MALL):
+    the Q4_K FFN up/down pair, the Q8_0 matvec 4864x896, the q8-KV
+    flash-decode (32 q / 8 KV heads, D 128, n_kv 8192, batch 1), the prefill matmuls and
     the causal prefill attention. Per-call time from HIP events on the launch stream (graph replay
     and direct launches; with `eager`, direct launches only)."""
     out = {}
@@ -557,7 +557,7 @@ def extra_workloads(dev, ev, stream, n: int, eager: bool = False) -> dict:
         ev.record(b, stream)
         return ev.elapsed_ms(a, b) / nn
 
-    # configs[1]: the Llama-3-8B FFN up / down Q4_K matvec pair
+    # the Llama-3-8B FFN up / down Q4_K matvec pair
     N_up, K_up, N_dn, K_dn = 14336, 4096, 4096, 14336
     up_blocks = S.quant_rows(1, S.seed_of("cfg2", "w_up"), N_up, K_up)
     dn_blocks = S.quant_rows(1, S.seed_of("cfg2", "w_down"), N_dn, K_dn)
@@ -584,7 +584,7 @@ def extra_workloads(dev, ev, stream, n: int, eager: bool = False) -> dict:
         "copies": copies}
     del ups, dns
 
-    # configs[0]: Q8_0 4864 x 896
+    # Q8_0 4864 x 896
     N, K = 4864, 896
     blocks = S.quantize_q8_0(S.normal(S.seed_of("cfg1", "w"), N * K, 0.02).reshape(N, K))
     per = blocks.nbytes
@@ -601,7 +601,7 @@ def extra_workloads(dev, ev, stream, n: int, eager: bool = False) -> dict:
                                    "copies": copies}
     del ws
 
-    # configs[2]: flash-decode over a q8_0 KV cache
+    # flash-decode over a q8_0 KV cache
     n_head, n_kv_head, D, n_kv = 32, 8, 128, 8192
     E = n_kv_head * D
     kf = dev.upload(S.normal(S.seed_of("cfg3", "k"), n_kv * E))
@@ -654,7 +654,7 @@ def extra_workloads(dev, ev, stream, n: int, eager: bool = False) -> dict:
     plan.free()
     del caches
 
-    # configs[3]: prefill at Llama-3-8B shapes, 512 tokens: Q8_0 MUL_MAT on the int8 matrix cores
+    # prefill at Llama-3-8B shapes, 512 tokens: Q8_0 MUL_MAT on the int8 matrix cores
     T, K = 512, 4096
     xq = dev.upload(S.normal(S.seed_of("cfg4", "x"), T * K))
     for name, N in (("prefill_q8_0_512x4096x4096", 4096), ("prefill_q8_0_512x14336x4096", 14336)):
@@ -686,7 +686,7 @@ def extra_workloads(dev, ev, stream, n: int, eager: bool = False) -> dict:
                      "launches_per_call": 2, "note": "QACT A256 of the 512 rows + the Q4_K matrix-core kernel"}
         del ws, yb, x4
 
-    # configs[3]: causal flash attention over 512 tokens (32 q / 8 KV heads, D 128, q8_0 KV); the
+    # causal flash attention over 512 tokens (32 q / 8 KV heads, D 128, q8_0 KV); the
     # work list of 512 rows is copied to the device per call, so this one is timed eagerly
     T, n_head, n_kv_head, D = 512, 32, 8, 128
     E = n_kv_head * D
@@ -769,7 +769,7 @@ def pmc_child(reps: int = 3) -> int:
     return 0
 
 
-# BASELINE configs[0]-[2] in the configs counter child: (name, kernel substring, algorithmic bytes per launch)
+# the decode workloads in the counter child: (name, kernel substring, algorithmic bytes per launch)
 PMC_CONFIGS = [("q8_0_matvec_4864x896", "k_mv_q80", 4864 * 28 * 34 + 4 * 896 + 4 * 4864),
                ("q4k_up_14336x4096", "k_mv_q4k", 14336 * 16 * 144 + 4 * 4096 + 4 * 14336),
                ("q4k_down_4096x14336", "k_mv_q4k", 4096 * 56 * 144 + 4 * 14336 + 4 * 4096),
@@ -777,7 +777,7 @@ PMC_CONFIGS = [("q8_0_matvec_4864x896", "k_mv_q80", 4864 * 28 * 34 + 4 * 896 + 4
 
 
 def pmc_configs_child(reps: int = 3) -> int:
-    """Counter child for BASELINE configs[0]-[2] (run under rocprofv3 --pmc): the calibration copy, then
+    """Counter child for the decode workloads (run under rocprofv3 --pmc): the calibration copy, then
     `reps` launches each, over device copies that rotate (no launch finds its bytes in a cache the one
     before filled), of the Q8_0 matvec 4864 x 896, the Q4_K up 14336 x 4096 and down 4096 x 14336
     matvecs, and the planned FLASH_ATTN_EXT decode at 8192 cells (one k_fa_dec launch), with the seeds
@@ -831,7 +831,7 @@ def pmc_configs_child(reps: int = 3) -> int:
 
 
 def measure_config_traffic(reps: int = 3) -> dict:
-    """HBM bytes per launch of the configs[0]-[2] kernels: FETCH_SIZE and WRITE_SIZE (two rocprofv3
+    """HBM bytes per launch of the decode workloads' kernels: FETCH_SIZE and WRITE_SIZE (two rocprofv3
     --pmc passes over the configs child), each scaled by the counter's reading for the calibration copy;
     with each kernel's algorithmic bytes and their ratio."""
     if shutil.which("rocprofv3") is None:
@@ -893,7 +893,7 @@ PREFILL_PMC = [("q8_0 512x4096x4096", 0, 4096, 4096, 0), ("q4_K 512x4096x14336",
 
 
 def pmc_prefill_child(reps: int = 2) -> int:
-    """Counter child for the prefill matmuls of BASELINE configs[3]: `reps` launches each of the Q8_0
+    """Counter child for the prefill matmuls: `reps` launches each of the Q8_0
     512x4096x4096, Q4_K 512x4096x14336 and Q4_K + GLU 512x28672x4096 MUL_MATs (activation QACT kernel +
     matrix-core kernel), in that order."""
     dev = tsr_hip.Device(0)
@@ -975,7 +975,7 @@ def main() -> int:
     ap.add_argument("--steps", type=int, default=128, help="timed decode tokens")
     ap.add_argument("--warmup", type=int, default=8, help="untimed decode tokens before them (>= 2)")
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline leg")
-    ap.add_argument("--no-extra", action="store_true", help="skip the other BASELINE configs")
+    ap.add_argument("--no-extra", action="store_true", help="skip the other workloads")
     ap.add_argument("--no-traffic", action="store_true", help="skip the rocprofv3 --pmc traffic passes")
     ap.add_argument("--eager", action="store_true",
                     help="time everything as direct launches: no HIP graph is built (so the adapter leg, which "
@@ -1051,7 +1051,7 @@ def main() -> int:
         also["adapter_decode_llama3_8b_q4k"] = adapter
     cpu = None if args.no_cpu else cpu_decode(e2e)
     if cpu is not None:
-        print("bench: CPU baselines of configs[0]-[3]", file=sys.stderr, flush=True)
+        print("bench: CPU baselines of the single-op workloads", file=sys.stderr, flush=True)
         cpu["per_config"] = cpu_configs(cpu["cores"])
     ms_tok = e2e["ms_per_token"]
     out = {

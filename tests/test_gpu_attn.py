@@ -25,7 +25,7 @@ def _cache(oc, kv_size, E, seed):
 def _fa(dev, oc, n_kv, kv_size, n_head, n_head_kv, D, T=1, mask=None, new_runs=None, seed=3, q=None):
     E = n_head_kv * D
     kc, vc = _cache(oc, kv_size, E, seed)
-    if q is None:   # Q drawn as f16 N(0, 1) and widened exactly (BASELINE configs[2])
+    if q is None:   # Q drawn as f16 N(0, 1) and widened exactly
         q = S.normal(seed + 2, T * n_head * D).reshape(T, n_head * D).astype(np.float16).astype(np.float32)
     mask = np.zeros((T, n_kv), np.float16) if mask is None else mask
     scale = np.float32(1.0 / math.sqrt(D))
@@ -43,7 +43,7 @@ def _fa(dev, oc, n_kv, kv_size, n_head, n_head_kv, D, T=1, mask=None, new_runs=N
 
 
 def test_fa_decode_baseline_shape(dev, oc):
-    """BASELINE configs[2]: 32 q heads, 8 KV heads, D 128, n_kv 8192, batch 1."""
+    """32 q heads, 8 KV heads, D 128, n_kv 8192, batch 1."""
     got, want = _fa(dev, oc, 8192, 8192, 32, 8, 128)
     assert np.abs(got - want).max() <= 2e-3
     assert_bits_equal(got, want, "fa decode 8192")
@@ -72,7 +72,7 @@ def test_fa_causal_prefill(dev, oc):
 
 
 def test_fa_causal_prefill_baseline_512(dev, oc):
-    """causal flash attention over a 512-token ubatch at cells 0 .. 511, 32 q / 8 KV
+    """Causal flash attention over a 512-token ubatch at cells 0 .. 511, 32 q / 8 KV
     heads, D 128, q8_0 K / V, Q drawn f16 N(0, 1): row t sees cells [0, t], the ubatch's cells newest
     last. Every output of every row bit-exact (the contract allows 2e-3 absolute, asserted too)."""
     T = 512

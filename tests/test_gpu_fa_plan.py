@@ -1,5 +1,5 @@
 """GPU parity of the planned FLASH_ATTN_EXT decode entry point (tsr_hip_flash_attn_plan: one launch of the
-decode form, k_fa_dec) against the CPU oracle, at the BASELINE shape and beyond: every chunk count that
+decode form, k_fa_dec) against the CPU oracle, at the 8192-cell shape and beyond: every chunk count that
 makes the reducers run one, two or three rounds of items, bit for bit. Also the tag wrap of the form's
 exchanges and the counter that names the form that ran."""
 import math
@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 
 def _case(dev, oc, n_kv, n_head=32, n_head_kv=8, D=128, kv_size=None, seed=None):
-    """BASELINE configs[2]'s draws: K, V f32 N(0, 1) through SET_ROWS (QACT A32) into q8_0 caches, Q f16
+    """The decode attention workload's draws: K, V f32 N(0, 1) through SET_ROWS (QACT A32) into q8_0 caches, Q f16
     N(0, 1) widened exactly, scale 1/sqrt(D), a mask of zeros over n_kv cells (one FAST run)."""
     kv_size = kv_size or n_kv
     E = n_head_kv * D
@@ -43,7 +43,7 @@ def _free(c):
 
 # 2048-cell chunks at this shape (NCG 128 groups); the reducers load 3 items per round
 @pytest.mark.parametrize("n_kv", [
-    8192,    # BASELINE configs[2]: 4 chunks, two reducer rounds (3 + 1)
+    8192,    # 4 chunks, two reducer rounds (3 + 1)
     6200,    # 4 chunks, the last one short
     12288,   # 6 chunks: two full rounds
     13000,   # 7 chunks: two full rounds and a partial one

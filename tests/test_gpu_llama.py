@@ -169,7 +169,7 @@ def test_prefill_refusals(dev):
 
 
 def test_decode_llama3_8b_token_matches_oracle(dev, oc):
-    """BASELINE configs[4] at its full shape: the Llama-3-8B-architecture Q4_K model (32 layers, n_embd
+    """The e2e decode at its full shape: the Llama-3-8B-architecture Q4_K model (32 layers, n_embd
     4096, n_ff 14336, 32 q / 8 KV heads of 128, vocabulary 128256), q8_0 caches holding a short history,
     one decode token eagerly and the same token by graph replay (the form the bench times): all 128256
     logits bit-equal to the oracle composition's step, and the same greedy token."""

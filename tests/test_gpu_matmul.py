@@ -4,7 +4,7 @@ ABI against the CPU oracle: bit-exact f32 outputs, as for the matvec path.
 The prefill path quantizes every token row (QACT A32), takes the integer block sums from the i8
 matrix core and the scale products from the f32 matrix core; these tests cover ragged tiles (T and
 N not multiples of 64), every K class (one block, under 16 blocks, many rounds of the 16 partials),
-the fused addend / accumulate flags, special activations and weight scales, and the BASELINE
+the fused addend / accumulate flags, special activations and weight scales, and the benchmark's
 prefill shape (512 tokens x 4096 x 4096) on a sample of tokens and rows."""
 import numpy as np
 import pytest
@@ -61,7 +61,7 @@ def test_mm_q8_0_specials(dev, oc):
 
 
 def test_mm_q8_0_baseline_prefill_shape(dev, oc):
-    """BASELINE configs[3] (512 tokens x W[4096 x 4096] Q8_0): every output of a sample of tokens,
+    """The benchmark's prefill (512 tokens x W[4096 x 4096] Q8_0): every output of a sample of tokens,
     and every token of a sample of rows."""
     T, N, K = 512, 4096, 4096
     blocks = S.quantize_q8_0(S.normal(S.seed_of("cfg4", "w_q"), N * K, 0.02).reshape(N, K))
@@ -77,7 +77,7 @@ def test_mm_q8_0_baseline_prefill_shape(dev, oc):
 
 
 def test_mm_q8_0_baseline_prefill_ffn_shape(dev, oc):
-    """BASELINE configs[3] (512 tokens x W[14336 x 4096] Q8_0, the FFN up shape): every output of a
+    """The benchmark's prefill (512 tokens x W[14336 x 4096] Q8_0, the FFN up shape): every output of a
     sample of tokens, and every token of a sample of rows (first, middle and last row blocks)."""
     T, N, K = 512, 14336, 4096
     blocks = S.quantize_q8_0(S.normal(S.seed_of("cfg4", "w_14336"), N * K, 0.02).reshape(N, K))
